@@ -82,22 +82,41 @@ __device__ __forceinline__ void wave_sync()
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// Inclusive scans over the wave by data-parallel-primitive moves (row shifts
+// inside the 16-lane rows, then the row ends broadcast to the later rows): one
+// VALU instruction per step, where a shuffle goes through the LDS unit.  Every
+// lane of the wave must be active.
+template <int kCtrl, int kRows>
+__device__ __forceinline__ uint32_t dpp_or_zero(uint32_t v)
+{
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, kCtrl, kRows, 0xF, false);
+}
+
 __device__ __forceinline__ uint32_t wave_incl_scan(uint32_t v)
 {
-    const int lane = (int)__lane_id();
-#pragma unroll
-    for (int d = 1; d < kWave; d <<= 1) {
-        const uint32_t t = __shfl_up(v, d, kWave);
-        if (lane >= d) v += t;
-    }
+    v += dpp_or_zero<0x111, 0xF>(v);    // row_shr:1
+    v += dpp_or_zero<0x112, 0xF>(v);
+    v += dpp_or_zero<0x114, 0xF>(v);
+    v += dpp_or_zero<0x118, 0xF>(v);    // row_shr:8
+    v += dpp_or_zero<0x142, 0xA>(v);    // row_bcast:15 into rows 1 and 3
+    v += dpp_or_zero<0x143, 0xC>(v);    // row_bcast:31 into rows 2 and 3
+    return v;
+}
+
+__device__ __forceinline__ uint32_t wave_incl_max(uint32_t v)
+{
+    v = max(v, dpp_or_zero<0x111, 0xF>(v));
+    v = max(v, dpp_or_zero<0x112, 0xF>(v));
+    v = max(v, dpp_or_zero<0x114, 0xF>(v));
+    v = max(v, dpp_or_zero<0x118, 0xF>(v));
+    v = max(v, dpp_or_zero<0x142, 0xA>(v));
+    v = max(v, dpp_or_zero<0x143, 0xC>(v));
     return v;
 }
 
 __device__ __forceinline__ uint32_t wave_sum(uint32_t v)
 {
-#pragma unroll
-    for (int d = kWave / 2; d >= 1; d >>= 1) v += __shfl_xor(v, d, kWave);
-    return v;
+    return (uint32_t)__builtin_amdgcn_readlane((int)wave_incl_scan(v), kWave - 1);
 }
 
 __device__ __forceinline__ float wave_min(float v)

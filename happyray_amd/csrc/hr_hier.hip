@@ -85,6 +85,7 @@ __device__ __forceinline__ GridRegs inst_grid_regs(const InstGrid& q)
     g.rx = q.res[0];
     g.ry = q.res[1];
     g.rz = q.res[2];
+    g.small = false;
     return g;
 }
 
@@ -808,8 +809,8 @@ template <class Gen>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) void k_hier_persist_bt(HierScene H, Gen g, uint32_t* __restrict__ pool,
                                                             uint32_t refill, unsigned long long* ray_count)
 {
-    __shared__ WaveTests<kBatchK> lds[kBlock / kWave];
-    WaveTests<kBatchK>& W = lds[__builtin_amdgcn_readfirstlane((int)threadIdx.x) / kWave];
+    __shared__ WaveTests lds[kBlock / kWave];
+    WaveTests& W = lds[__builtin_amdgcn_readfirstlane((int)threadIdx.x) / kWave];
     const GridRegs G = load_grid(H.top);
     const uint32_t lane = __lane_id();
     const uint64_t lt = __lanemask_lt();
@@ -844,12 +845,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
             bool entered = false;
             done = hp_unit(H, G, r, entered);
             if (entered) {
-                W.ox[lane] = r.ot.x;
-                W.oy[lane] = r.ot.y;
-                W.oz[lane] = r.ot.z;
-                W.dx[lane] = r.dt.x;
-                W.dy[lane] = r.dt.y;
-                W.dz[lane] = r.dt.z;
+                W.set_ray(lane, r.ot, r.dt, r.rayT);
             }
         }
         wave_test_range<false, kBatchK>(H.rec, H.prims, W, r.pit, r.pend, r.rayT, r.hit, lane, live && !done, wk);

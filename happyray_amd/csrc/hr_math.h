@@ -58,6 +58,38 @@ HR_HD float len(f3 a) { return sqrtf(dot(a, a)); }
 HR_HD f3 normalize(f3 a) { return a * (1.f / sqrtf(dot(a, a))); }
 HR_HD float get(f3 a, int i) { return i == 0 ? a.x : (i == 1 ? a.y : a.z); }
 
+// 1 / x correctly rounded, as the division gives it, for 2^-125 <= |x| <= 2^125
+// (every such x was compared with the division): the hardware estimate and one
+// fused Newton step instead of the division's scaling and fix-up.
+__device__ __forceinline__ float rcp_in_range(float x)
+{
+    const float y = __builtin_amdgcn_rcpf(x);
+    return __builtin_fmaf(__builtin_fmaf(-x, y, 1.f), y, y);
+}
+
+constexpr float kRcpLow = 0x1p-125f, kRcpHigh = 0x1p125f;
+
+__device__ __forceinline__ float rcp_rn(float x)
+{
+    float y = rcp_in_range(x);
+    if (!(fabsf(x) >= kRcpLow && fabsf(x) <= kRcpHigh)) y = 1.f / x;
+    return y;
+}
+
+// a / b correctly rounded from y = 1 / b correctly rounded (Markstein, IBM J.
+// Res. Dev. 34(1), 1990: the residual of a quotient within one unit in the last
+// place, formed by a fused multiply-add, rounds it correctly; the first step
+// brings the quotient there).  For |b| in [2^-60, 2^60] and a either 0 or in
+// [2^-60, 2^60], where no step leaves the normal range.
+__device__ __forceinline__ float div_by_rcp(float a, float b, float y)
+{
+    float q = a * y;
+    q = __builtin_fmaf(__builtin_fmaf(-b, q, a), y, q);
+    return __builtin_fmaf(__builtin_fmaf(-b, q, a), y, q);
+}
+
+constexpr float kDivLow = 0x1p-60f, kDivHigh = 0x1p60f;
+
 // getLocalCoordinates (src/Core/Algebra.hpp:281-298), tangent scaled by
 // 1/(n_c0^2 + n_z^2) exactly as the reference writes it.
 HR_HD void local_frame(f3 n, f3& t, f3& b)

@@ -230,8 +230,8 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(6))) voi
     unsigned long long* ray_count, unsigned long long* stats)
 {
     if (gen.skipped()) return;
-    __shared__ WaveTests<kK> lds[kBlock / kWave];
-    WaveTests<kK>& W = lds[__builtin_amdgcn_readfirstlane((int)threadIdx.x) / kWave];
+    __shared__ WaveTests lds[kBlock / kWave];
+    WaveTests& W = lds[__builtin_amdgcn_readfirstlane((int)threadIdx.x) / kWave];
     const GridRegs G = load_grid(S.gp);
     const uint32_t lane = __lane_id();
     const uint64_t lt = __lanemask_lt();
@@ -255,12 +255,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(6))) voi
                     started += ok ? 1u : 0u;
                     live = ok && ray_begin<kTwo, kAny>(G, S, r, wk);
                     if (live) {
-                        W.ox[lane] = r.org.x;
-                        W.oy[lane] = r.org.y;
-                        W.oz[lane] = r.org.z;
-                        W.dx[lane] = r.dir.x;
-                        W.dy[lane] = r.dir.y;
-                        W.dz[lane] = r.dir.z;
+                        W.set_ray(lane, r.org, r.dir, r.t);
                     } else {
                         gen.finish(j, r, ok, S);
                     }
@@ -273,6 +268,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(6))) voi
         }
         bool done = false;
         if (live && r.it >= r.end) {
+#pragma unroll 1
             for (uint32_t m = 0; m < steps_max; ++m) {
                 if (kTwo) {
                     bool top = true;
@@ -283,18 +279,18 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(6))) voi
                             done = k != 1;
                         }
                     }
-                    if (top) done = !top_step(G, S, r, mk(W.ox[lane], W.oy[lane], W.oz[lane]), wk);
+                    if (top) done = !top_step(G, S, r, W.org(lane), W.dir(lane), wk);
                 } else {
                     done = !advance_uniform<kAny>(G, S, r, wk);
                 }
                 if (done || r.it < r.end) break;
             }
         }
-        if (wave_test_batch<kAny>(S, W, r, lane, live && !done, wk)) done = true;
+        if (wave_test_batch<kAny, kK>(S, W, r, lane, live && !done, wk)) done = true;
         if (live && done) {
             live = false;
-            r.org = mk(W.ox[lane], W.oy[lane], W.oz[lane]);
-            r.dir = mk(W.dx[lane], W.dy[lane], W.dz[lane]);
+            r.org = W.org(lane);
+            r.dir = W.dir(lane);
             gen.finish(j, r, true, S);
         }
     }
@@ -411,11 +407,11 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5))) voi
     uint32_t nb, uint32_t nrays, uint32_t* __restrict__ pool, uint32_t refill, uint32_t steps_max,
     unsigned long long* ray_count, unsigned long long* stats)
 {
-    __shared__ WaveTests<kBatchK> lds[kBlock / kWave];
+    __shared__ WaveTests lds[kBlock / kWave];
     __shared__ const float4* recs[kBlock];
     __shared__ const uint32_t* prims[kBlock];
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)threadIdx.x) / kWave;
-    WaveTests<kBatchK>& W = lds[wave];
+    WaveTests& W = lds[wave];
     const float4* const* own_rec = recs + wave * kWave;
     const uint32_t* const* own_prims = prims + wave * kWave;
     const uint32_t lane = __lane_id();
@@ -458,12 +454,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5))) voi
                     live = ray_begin<true, kAny>(G, S, r, wk);
                     j = jl;
                     if (live) {
-                        W.ox[lane] = r.org.x;
-                        W.oy[lane] = r.org.y;
-                        W.oz[lane] = r.org.z;
-                        W.dx[lane] = r.dir.x;
-                        W.dy[lane] = r.dir.y;
-                        W.dz[lane] = r.dir.z;
+                        W.set_ray(lane, r.org, r.dir, r.t);
                         recs[threadIdx.x] = S.rec;
                         prims[threadIdx.x] = S.prims;
                     } else if (kAny) {
@@ -483,6 +474,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5))) voi
         }
         bool done = false;
         if (live && r.it >= r.end) {
+#pragma unroll 1
             for (uint32_t m = 0; m < steps_max; ++m) {
                 bool top = true;
                 if (r.in_leaf) {
@@ -492,7 +484,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5))) voi
                         done = k != 1;
                     }
                 }
-                if (top) done = !top_step(G, S, r, mk(W.ox[lane], W.oy[lane], W.oz[lane]), wk);
+                if (top) done = !top_step(G, S, r, W.org(lane), W.dir(lane), wk);
                 if (done || r.it < r.end) break;
             }
         }
@@ -510,8 +502,8 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5))) voi
                 B.t_out[j] = r.t;
                 B.prim_out[j] = r.t < kFltMax ? r.best - D.tri_base : D.nt;
                 if (B.hits) {
-                    r.org = mk(W.ox[lane], W.oy[lane], W.oz[lane]);
-                    r.dir = mk(W.dx[lane], W.dy[lane], W.dz[lane]);
+                    r.org = W.org(lane);
+                    r.dir = W.dir(lane);
                     store_hit(B.hits, B.n, j, r);
                 }
             }

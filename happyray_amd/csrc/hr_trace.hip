@@ -112,8 +112,8 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(6))) voi
     uint32_t* __restrict__ hit_prims, uint32_t steps_max, unsigned long long* ray_count)
 {
     if (frame_skipped(ra)) return;
-    __shared__ WaveTests<kBatchK> lds[kBlock / kWave];
-    WaveTests<kBatchK>& W = lds[__builtin_amdgcn_readfirstlane((int)threadIdx.x) / kWave];
+    __shared__ WaveTests lds[kBlock / kWave];
+    WaveTests& W = lds[__builtin_amdgcn_readfirstlane((int)threadIdx.x) / kWave];
     const uint32_t pix = blockIdx.x * blockDim.x + threadIdx.x;   // row order: tiles measured slower here
     const bool active = pix < npix;
     count_rays(ray_count, active);
@@ -124,7 +124,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(6))) voi
     const f3 org = mk(cam.center[0], cam.center[1], cam.center[2]);
     float t = kFltMax;
     f3 dir;
-    const uint32_t best = trace_wave<kTwo, false>(G, S, W, active, org, d0, t, dir, steps_max, wk);
+    const uint32_t best = trace_wave<kTwo, false, kBatchK>(G, S, W, active, org, d0, t, dir, steps_max, wk);
     if (active) {
         const uint32_t prim = t < kFltMax ? best : S.nt;
         const f3 hp = org + (t - kEps) * dir;
@@ -261,9 +261,9 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
                                                     unsigned long long* ray_count)
 {
     if (frame_skipped(ra)) return;
-    __shared__ WaveTests<kBatchK> lds[kBlock / kWave];
+    __shared__ WaveTests lds[kBlock / kWave];
     __shared__ float light_terms[6][kBlock];   // a vertex's light terms wait here across its shadow ray
-    WaveTests<kBatchK>& W = lds[__builtin_amdgcn_readfirstlane((int)threadIdx.x) / kWave];
+    WaveTests& W = lds[__builtin_amdgcn_readfirstlane((int)threadIdx.x) / kWave];
     const uint32_t pix = blockIdx.x * blockDim.x + threadIdx.x;
     const bool in = pix < npix;
     const GridRegs G = load_grid(S.gp);
@@ -307,7 +307,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
         // the shadow ray (PathTracer.h:236-258) and its light term
         float st = 0.9999f;
         f3 dd;
-        trace_wave<kTwo, true>(G, S, W, shadow, P.org, V.sdir, st, dd, steps_max, wk);
+        trace_wave<kTwo, true, kBatchK>(G, S, W, shadow, P.org, V.sdir, st, dd, steps_max, wk);
         if (shadow) {
             ++traced;
             if (!(st < 0.9999f)) {
@@ -321,7 +321,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
         // the extension ray (PathTracer.h:318-332)
         float t = kFltMax;
         f3 d2;
-        const uint32_t hit = trace_wave<kTwo, false>(G, S, W, alive, P.org, P.dir, t, d2, steps_max, wk);
+        const uint32_t hit = trace_wave<kTwo, false, kBatchK>(G, S, W, alive, P.org, P.dir, t, d2, steps_max, wk);
         if (alive) {
             ++traced;
             P.dir = d2;

@@ -19,6 +19,7 @@ typedef __attribute__((address_space(3))) const float* lds_cfloat_ptr;
 struct GridRegs {
     f3 bmin, bmax, cs, csr;
     int rx, ry, rz;
+    bool small;           // a cell's index by 24-bit multiplies: rx and ry * rz below 2^24
     lds_cfloat_ptr sub;   // nullptr, or the workgroup's table of leaf cell sizes (sub_table)
 };
 
@@ -60,6 +61,7 @@ __device__ __forceinline__ GridRegs load_grid(const GridParams* gp)
     g.rx = gp->res[0];
     g.ry = gp->res[1];
     g.rz = gp->res[2];
+    g.small = (uint32_t)g.rx < (1u << 24) && (uint64_t)(uint32_t)g.ry * (uint32_t)g.rz < (1ull << 24);
     return g;
 }
 

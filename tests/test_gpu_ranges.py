@@ -1,0 +1,43 @@
+"""Ray queries where the traversal's short forms meet their limits, against the
+oracle bit for bit: scenes and directions scaled by powers of two beyond the
+ranges of the short reciprocals and quotients (the full divisions take over),
+axis-parallel rays (infinite reciprocals), origins on cell planes, and ray
+counts about a wave and a workgroup."""
+import numpy as np
+import pytest
+
+import pyoracle as O
+from gpu_util import gpu_engine, oracle_grid, random_rays
+from happyray_amd import GRID_TWO_LEVEL, GRID_UNIFORM, GRID_UNIFORM_EXACT, scenes
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("mesh_exp,dir_exp", [(0, 0), (0, -70), (0, 60), (-35, -35), (-35, -55), (30, 30),
+                                              (42, 42)])
+@pytest.mark.parametrize("kind,lt,ll", [(GRID_TWO_LEVEL, 0.25, 2.2), (GRID_UNIFORM, 5.0, 1.0),
+                                        (GRID_UNIFORM_EXACT, 5.0, 1.0)])
+def test_scaled_scenes_and_directions(kind, lt, ll, mesh_exp, dir_exp):
+    sc = scenes.random_soup(5, 3000, extent=8.0, size=0.6)
+    org, d = random_rays(sc, 4096, seed=6)
+    # some origins on the planes of an 8-cell lattice through the scene
+    org[:, :256] = np.round(org[:, :256])
+    sc.verts = np.ldexp(sc.verts, mesh_exp).astype(np.float32)
+    org = np.ldexp(org, mesh_exp).astype(np.float32)
+    d = np.ldexp(d, dir_exp).astype(np.float32)
+    e = gpu_engine(sc, kind, lt, ll)
+    og = oracle_grid(sc, kind, lt, ll)
+    tmax = float(np.float32(np.ldexp(2.0, mesh_exp - dir_exp)))
+    for n in (1, 63, 65, 1023, 4096):
+        o, q = org[:, -n:], d[:, -n:]      # the last rays are the axis-parallel ones
+        t_o, p_o, _ = O.trace(og, o, q)
+        s_o, _, _ = O.trace(og, o, q, anyhit=True, tmax=tmax)
+        for batch in (1, 0):
+            e.set_tuning(test_batch=batch)
+            t, p = e.trace(o, q)
+            np.testing.assert_array_equal(t.view(np.uint32), t_o.view(np.uint32))
+            np.testing.assert_array_equal(p, p_o)
+            np.testing.assert_array_equal(e.occluded(o, q, tmax), (s_o < tmax).astype(np.uint8))
+    if (mesh_exp, dir_exp) in ((0, 0), (0, -70), (-35, -35), (-35, -55), (30, 30)):
+        assert (p_o < sc.nt).mean() > 0.5   # the scaled rays do hit
+    e.close()
