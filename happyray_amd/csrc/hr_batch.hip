@@ -275,10 +275,13 @@ hr_status do_build(hr_batch* b)
                 return fail(HR_ERR_CAPACITY, "grid resolution too large");
             b->cells_cap = grow(b->cells_cap, st.num_cells);
         } else if (st.overflow & hr::kOverflowPairs) {
+            if (st.num_pairs == 0xFFFFFFFFu) return fail(HR_ERR_CAPACITY, "the grids need 2^32 entries or more");
             b->pairs_cap = grow(b->pairs_cap, st.num_pairs);
         } else if (st.overflow & hr::kOverflowLeaves) {
+            if (st.num_leaves == 0xFFFFFFFFu) return fail(HR_ERR_CAPACITY, "the grids need 2^32 entries or more");
             b->leaves_cap = grow(b->leaves_cap, st.num_leaves);
         } else if (st.overflow & hr::kOverflowLeafPairs) {
+            if (st.num_leaf_pairs == 0xFFFFFFFFu) return fail(HR_ERR_CAPACITY, "the grids need 2^32 entries or more");
             b->leaf_pairs_cap = grow(b->leaf_pairs_cap, st.num_leaf_pairs);
         }
     }

@@ -103,6 +103,21 @@ __device__ __forceinline__ uint32_t wave_incl_scan(uint32_t v)
     return v;
 }
 
+// a + b, or the largest value where the sum does not fit: sums of counts keep
+// "too many" too many instead of wrapping to a small total
+__device__ __forceinline__ uint32_t add_sat(uint32_t a, uint32_t b) { return __builtin_elementwise_add_sat(a, b); }
+
+__device__ __forceinline__ uint32_t wave_incl_scan_sat(uint32_t v)
+{
+    v = add_sat(v, dpp_or_zero<0x111, 0xF>(v));
+    v = add_sat(v, dpp_or_zero<0x112, 0xF>(v));
+    v = add_sat(v, dpp_or_zero<0x114, 0xF>(v));
+    v = add_sat(v, dpp_or_zero<0x118, 0xF>(v));
+    v = add_sat(v, dpp_or_zero<0x142, 0xA>(v));
+    v = add_sat(v, dpp_or_zero<0x143, 0xC>(v));
+    return v;
+}
+
 __device__ __forceinline__ uint32_t wave_incl_max(uint32_t v)
 {
     v = max(v, dpp_or_zero<0x111, 0xF>(v));
@@ -116,7 +131,7 @@ __device__ __forceinline__ uint32_t wave_incl_max(uint32_t v)
 
 __device__ __forceinline__ uint32_t wave_sum(uint32_t v)
 {
-    return (uint32_t)__builtin_amdgcn_readlane((int)wave_incl_scan(v), kWave - 1);
+    return (uint32_t)__builtin_amdgcn_readlane((int)wave_incl_scan_sat(v), kWave - 1);
 }
 
 __device__ __forceinline__ float wave_min(float v)

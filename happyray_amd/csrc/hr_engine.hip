@@ -612,6 +612,9 @@ void release_lane(hr_ctx::LaneFields& o)
     o.stream = nullptr;
 }
 
+// a saturated count (see the scan): no buffer can hold it
+constexpr char kTooMany[] = "the grid needs 2^32 entries or more";
+
 hr_status do_build(hr_ctx* c)
 {
     if (!c->src1 || c->nv == 0) return fail(HR_ERR_STATE, "no geometry uploaded");
@@ -658,10 +661,13 @@ hr_status do_build(hr_ctx* c)
             if (st.num_cells == 0xFFFFFFFFu) return fail(HR_ERR_CAPACITY, "grid resolution too large");
             c->cells_cap = grow(c->cells_cap, st.num_cells);
         } else if (st.overflow & hr::kOverflowPairs) {
+            if (st.num_pairs == 0xFFFFFFFFu) return fail(HR_ERR_CAPACITY, kTooMany);
             c->pairs_cap = grow(c->pairs_cap, st.num_pairs);
         } else if (st.overflow & hr::kOverflowLeaves) {
+            if (st.num_leaves == 0xFFFFFFFFu) return fail(HR_ERR_CAPACITY, kTooMany);
             c->leaves_cap = grow(c->leaves_cap, st.num_leaves);
         } else if (st.overflow & hr::kOverflowLeafPairs) {
+            if (st.num_leaf_pairs == 0xFFFFFFFFu) return fail(HR_ERR_CAPACITY, kTooMany);
             c->leaf_pairs_cap = grow(c->leaf_pairs_cap, st.num_leaf_pairs);
         }
     }

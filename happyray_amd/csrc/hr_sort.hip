@@ -29,15 +29,15 @@ __device__ __forceinline__ uint32_t block_excl_scan(uint32_t v, uint32_t* lds_wa
 {
     const int lane = (int)__lane_id();
     const int w = (int)threadIdx.x / kWave;
-    const uint32_t inc = wave_incl_scan(v);
+    const uint32_t inc = wave_incl_scan_sat(v);
     if (lane == kWave - 1) lds_waves[w] = inc;
     __syncthreads();
     uint32_t off = 0;
     total = 0;
     for (int i = 0; i < (int)blockDim.x / kWave; ++i) {
         const uint32_t c = lds_waves[i];
-        if (i < w) off += c;
-        total += c;
+        if (i < w) off = add_sat(off, c);
+        total = add_sat(total, c);
     }
     __syncthreads();
     return off + inc - v;
@@ -49,7 +49,10 @@ __device__ __forceinline__ uint32_t block_excl_scan(uint32_t v, uint32_t* lds_wa
 
 // chain words: [0] tile counter, [1] epoch, [2..7] unused, then one 64-bit
 // flag per tile: epoch << 34 | status << 32 | value, status 1 = the tile's
-// sum, 2 = its inclusive prefix (0 = nothing published in this epoch)
+// sum, 2 = its inclusive prefix (0 = nothing published in this epoch).  Sums
+// saturate: a total past 32 bits stays above every capacity, so the check
+// refuses it (a wrapped one would pass, and the counted items overrun their
+// buffers)
 constexpr uint32_t kChainHead = 8;
 constexpr uint64_t kAggregate = 1, kPrefix = 2;
 constexpr int kSpinLimit = 1 << 16;
@@ -65,7 +68,7 @@ __device__ uint32_t tile_sum(const uint32_t* in, uint32_t tile, uint32_t n)
     uint32_t s = 0;
     const uint32_t b = tile * kScanTile;
     const uint32_t e = b + kScanTile < n ? b + kScanTile : n;
-    for (uint32_t i = b; i < e; ++i) s += in[i];
+    for (uint32_t i = b; i < e; ++i) s = add_sat(s, in[i]);
     return s;
 }
 
@@ -96,7 +99,7 @@ __global__ __launch_bounds__(kBlock) void k_scan_1p(const uint32_t* __restrict__
         for (int k = 0; k < kItems; ++k) {
             const uint32_t i = first + k;
             v[k] = i < n ? in[i] : 0u;
-            s += v[k];
+            s = add_sat(s, v[k]);
         }
         uint32_t agg;
         const uint32_t ex = block_excl_scan(s, lds, agg);
@@ -141,8 +144,8 @@ __global__ __launch_bounds__(kBlock) void k_scan_1p(const uint32_t* __restrict__
                     if ((ready & need) == need) {
                         uint32_t v = (lane <= last && p >= 0) ? val : 0u;
 #pragma unroll
-                        for (int d = kWave / 2; d >= 1; d >>= 1) v += __shfl_xor(v, d, kWave);
-                        excl += v;
+                        for (int d = kWave / 2; d >= 1; d >>= 1) v = add_sat(v, __shfl_xor(v, d, kWave));
+                        excl = add_sat(excl, v);
                         if (pre || p_hi - (kWave - 1) <= 0) break;
                         p_hi -= kWave;
                         spins = 0;
@@ -152,14 +155,14 @@ __global__ __launch_bounds__(kBlock) void k_scan_1p(const uint32_t* __restrict__
                     __builtin_amdgcn_s_sleep(1);
                 }
                 if (lane == 0)
-                    __hip_atomic_store(&flags[tile], flag_pack(epoch, kPrefix, excl + agg), __ATOMIC_RELAXED,
+                    __hip_atomic_store(&flags[tile], flag_pack(epoch, kPrefix, add_sat(excl, agg)), __ATOMIC_RELAXED,
                                        __HIP_MEMORY_SCOPE_AGENT);
             }
             if (lane == 0) {
                 s_excl = excl;
                 // the tile holding the last element knows the total
                 if ((n - 1) / kScanTile == tile) {
-                    const uint32_t total = excl + agg;
+                    const uint32_t total = add_sat(excl, agg);
                     if (total_dev) *total_dev = total;
                     if (check.st) {
                         if (total > check.cap) atomicOr(&check.st->overflow, check.bit);

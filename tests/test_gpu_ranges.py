@@ -8,7 +8,8 @@ import pytest
 
 import pyoracle as O
 from gpu_util import gpu_engine, oracle_grid, random_rays
-from happyray_amd import GRID_TWO_LEVEL, GRID_UNIFORM, GRID_UNIFORM_EXACT, scenes
+from happyray_amd import GRID_TWO_LEVEL, GRID_UNIFORM, GRID_UNIFORM_EXACT, HappyRayError, scenes
+from happyray_amd._lib import STATUS_NAMES
 
 pytestmark = pytest.mark.gpu
 
@@ -41,3 +42,16 @@ def test_scaled_scenes_and_directions(kind, lt, ll, mesh_exp, dir_exp):
     if (mesh_exp, dir_exp) in ((0, 0), (0, -70), (-35, -35), (-35, -55), (30, 30)):
         assert (p_o < sc.nt).mean() > 0.5   # the scaled rays do hit
     e.close()
+
+
+def test_leaf_counts_past_32_bits_are_refused():
+    """A cell volume so small that leaf density / volume overflows asks for 255^3
+    leaves in each of 729 cells: more than 2^32, which the build refuses."""
+    sc = scenes.random_soup(5, 3000, extent=8.0, size=0.6)
+    keep = sc.verts.copy()
+    sc.verts = np.ldexp(sc.verts, -42).astype(np.float32)
+    with pytest.raises(HappyRayError) as ex:
+        gpu_engine(sc, GRID_TWO_LEVEL, 0.25, 2.2)
+    assert STATUS_NAMES[ex.value.status] == "HR_ERR_CAPACITY"
+    sc.verts = keep
+    gpu_engine(sc, GRID_TWO_LEVEL, 0.25, 2.2).close()
