@@ -133,6 +133,25 @@ def test_batch_regrows_after_overflow():
     b.close()
 
 
+@pytest.mark.parametrize("tris", [[1], [21, 1, 1, 43, 85], [86] * 40, [1] * 300, [341, 342, 20, 683, 1, 40000],
+                                  [200000, 1, 150000]])
+def test_batch_bounds_of_runs(tris):
+    """Vertex runs that end at, before and past scene boundaries, many scenes in
+    one wave's 64 vertices, and scenes over many blocks.  Minima and maxima do
+    not round, so they are compared exactly."""
+    scs = [scenes.random_soup(500 + i, n, extent=10.0, size=0.4) for i, n in enumerate(tris)]
+    b = Batch()
+    b.set_scenes([(sc.verts, sc.idx) for sc in scs])
+    b.set_densities(0.25, 2.0)
+    b.build()
+    for s, sc in list(enumerate(scs))[:: max(1, len(scs) // 12)]:
+        bmin, bmax = O.bounds(sc.verts)
+        g = b.grid(s)[0]
+        np.testing.assert_array_equal(np.array(g.bmin[:], np.float32), bmin)
+        np.testing.assert_array_equal(np.array(g.bmax[:], np.float32), bmax)
+    b.close()
+
+
 def test_autotune_choice_keeps_results():
     scs = scene_set()[:6]
     b = Batch()
