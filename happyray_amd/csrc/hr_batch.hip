@@ -100,7 +100,7 @@ hr_status reserve_build(hr_batch* b)
     const uint32_t waves = cdiv(std::max<uint64_t>(std::max(b->nt, b->pairs_cap), 1), 64);
     const uint32_t waves_cap = (waves + 3) / 4 * 4 + 4;
     HR_TRY(b->wave_counts.reserve(waves_cap));
-    HR_TRY(b->wave_offsets.reserve(waves_cap));
+    HR_TRY(b->wave_offsets.reserve(hr::wave_offsets_words((uint32_t)b->wave_counts.cap, b->nt)));
     HR_TRY(b->keys.reserve(pair_max));
     HR_TRY(b->vals.reserve(pair_max));
     HR_TRY(b->keys_sorted.reserve(pair_max));

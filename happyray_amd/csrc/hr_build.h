@@ -22,7 +22,8 @@ struct BuildBuffers {
     BuildStatus* status;
     float4* rec;                // triangle records: 9 floats per triangle
     uint32_t* wave_counts;      // per-wave pair counts
-    uint32_t* wave_offsets;     // their exclusive scan
+    uint32_t* wave_offsets;     // their exclusive scan, then the list of waves with many candidates
+                                // (wave_offsets_words(waves_cap, nt) words)
     uint32_t* keys;             // unsorted keys / values (pairs, then leaf pairs)
     uint32_t* vals;
     uint32_t* keys_sorted;
@@ -61,6 +62,7 @@ struct SceneTable {
                                  // ranges clamp the first cell to res - 1 and the end to >= 1
 };
 
+size_t wave_offsets_words(uint32_t waves_cap, uint32_t nt);
 void launch_reset(BuildStatus* st, hipStream_t s);
 // fs != nullptr: the key frames are blocks fs->k1, fs->k2 of keys and the
 // coefficient is fs->coeff, all read on the device

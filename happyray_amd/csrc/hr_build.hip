@@ -53,7 +53,8 @@ __global__ void k_reset(BuildStatus* st)
         st->num_cells = st->num_pairs = st->num_leaves = st->num_leaf_pairs = 0u;
         st->overflow = 0u;
         st->n_pairs_eff = st->n_leaves_eff = st->n_leaf_pairs_eff = 0u;
-        st->pad[0] = st->pad[1] = 0u;
+        st->heavy = 0u;
+        st->pad = 0u;
     }
 }
 
@@ -259,6 +260,7 @@ struct WaveItems {
     int lo[3][kWave];
     int dx[kWave], dy[kWave];
     uint32_t excl[kWave];
+    uint32_t mark[kWave];
     uint32_t id[kWave];
     // exact insertion
     float v[9][kWave];
@@ -270,6 +272,45 @@ struct WaveItems {
     // scenes of a batch: per-owner grid width, z stride and first cell
     uint32_t gx[kWave], gz[kWave], cbase[kWave];
 };
+
+// owner of candidate j0 + lane of the wave's list (a lane owns the cnt
+// candidates from ex on): each lane marks its first place in the window, and a
+// maximum scan carries its number to its other places.  Two LDS accesses and
+// six moves where a binary search over the offsets takes six dependent reads.
+// Every lane of the wave calls it, with j0 below the total.
+__device__ __forceinline__ uint32_t list_owner(uint32_t* mark, uint32_t lane, uint32_t ex, uint32_t cnt, uint32_t j0)
+{
+    mark[lane] = 0u;
+    wave_sync();
+    if (cnt && ex < j0 + kWave && ex + cnt > j0) mark[ex > j0 ? ex - j0 : 0u] = lane;
+    wave_sync();
+    return wave_incl_max(mark[lane]);
+}
+
+// Waves of 64 triangles with many candidates (large triangles: walls, a ground)
+// are listed by the count pass and their candidates are spread over the launch
+// in kPairSlices slices each, in place of one wave that the whole launch waits
+// for.  A slice has at least kSliceMin candidates, so that reading the 64
+// triangles again is a small part of its work.  Two ground triangles of a
+// 74-cells-wide exact grid (82,000 triangles): the whole frame with its two passes
+// 1718 -> 645 us, 640 us a pass before; 768 wall
+// triangles of a two-level grid of 20,480: write pass 12.6 -> 5.1 us.
+constexpr uint32_t kPairsHeavy = 1024;     // candidates of a wave from which it is listed
+constexpr uint32_t kPairSlices = 32;
+constexpr uint32_t kSliceMin = 256;
+
+// the list in device memory: BuildStatus.heavy entries {wave, candidates}, and
+// for exact insertion the pairs of every slice
+struct PairList {
+    uint2* waves;
+    uint32_t* slice_pairs;
+};
+
+__device__ __forceinline__ uint32_t slice_len(uint32_t total)
+{
+    const uint32_t n = ((total + kPairSlices - 1u) / kPairSlices + kWave - 1u) / kWave * kWave;
+    return n < kSliceMin ? kSliceMin : n;
+}
 
 // scene of a global cell index: the last s with cell_base[s] <= c (cell
 // counts are positive, so the bases increase strictly)
@@ -284,136 +325,193 @@ __device__ __forceinline__ uint32_t scene_of(const uint32_t* base, uint32_t ns, 
     return lo;
 }
 
+// the passes of k_top_pairs: count, count the slices of the listed waves (exact
+// insertion), write
+constexpr int kPairsCount = 0, kPairsSlices = 1, kPairsWrite = 2;
+
 // kMulti: the triangles of a batch of scenes; each lane takes the grid of its
-// triangle's scene and writes global cell keys (cell_base of the scene + key)
-template <bool kExact, bool kWrite, bool kMulti = false>
+// triangle's scene and writes global cell keys (cell_base of the scene + key).
+// The first own_blocks workgroups take 64 consecutive triangles per wave; the
+// waves of the others take the slices of the listed waves in turn.
+template <bool kExact, int kPass, bool kMulti = false>
 __global__ __launch_bounds__(kBlock) void k_top_pairs(
     const uint32_t* __restrict__ idx, const float* __restrict__ vx, const float* __restrict__ vy,
     const float* __restrict__ vz, uint32_t nt, const GridParams* __restrict__ gp,
-    const BuildStatus* __restrict__ st, float4* __restrict__ rec, uint32_t* __restrict__ wave_counts,
+    BuildStatus* __restrict__ st, float4* __restrict__ rec, uint32_t* __restrict__ wave_counts,
     const uint32_t* __restrict__ wave_offsets, uint32_t* __restrict__ keys, uint32_t* __restrict__ vals,
-    uint32_t waves_cap, SceneTable T = SceneTable{}, uint2* __restrict__ zero = nullptr,
-    const uint32_t* __restrict__ zero_n = nullptr)
+    uint32_t waves_cap, uint32_t own_blocks, PairList list, SceneTable T = SceneTable{},
+    uint2* __restrict__ zero = nullptr, const uint32_t* __restrict__ zero_n = nullptr)
 {
     static_assert(!(kExact && kMulti), "batches use bounding-box insertion");
+    constexpr bool kWrite = kPass == kPairsWrite;
     __shared__ WaveItems sh[kWavesPerBlock];
     if (stop(st)) return;
     zero_cells(zero, zero_n);
     const int wl = (int)threadIdx.x / kWave;
-    const int lane = (int)__lane_id();
-    const uint32_t wg = blockIdx.x * kWavesPerBlock + (uint32_t)wl;
-    const uint32_t p = wg * kWave + (uint32_t)lane;
-    const bool valid = p < nt;
-    if (wg * kWave >= nt) {         // whole wave idle
+    const uint32_t lane = __lane_id();
+    WaveItems& W = sh[wl];
+    const bool own = blockIdx.x < own_blocks;
+    if (own && blockIdx.x * kWavesPerBlock * kWave + (uint32_t)wl * kWave >= nt) {         // whole wave idle
+        const uint32_t wg = blockIdx.x * kWavesPerBlock + (uint32_t)wl;
         if (!kWrite && lane == 0 && wg < waves_cap) wave_counts[wg] = 0u;
         return;
     }
 
-    uint32_t cbase = 0;
-    if (kMulti) {
-        const uint32_t sc = T.tri_scene[valid ? p : nt - 1u];
-        gp = T.gps + sc;
-        cbase = T.cell_base[sc];
-    }
-    const f3 bmin = mk(gp->bmin[0], gp->bmin[1], gp->bmin[2]);
-    const f3 cs = mk(gp->cs[0], gp->cs[1], gp->cs[2]);
-    const f3 csr = mk(gp->csr[0], gp->csr[1], gp->csr[2]);
-    const int rx = gp->res[0], ry = gp->res[1], rz = gp->res[2];
-
-    f3 v0 = rep(0.f), v1 = rep(0.f), v2 = rep(0.f);
-    uint32_t cnt = 0;
-    int mn[3] = { 0, 0, 0 }, mx[3] = { 0, 0, 0 };
-    if (valid) {
-        if (!kWrite) {
-            const uint32_t i0 = idx[3 * (size_t)p], i1 = idx[3 * (size_t)p + 1], i2 = idx[3 * (size_t)p + 2];
-            v0 = mk(vx[i0], vy[i0], vz[i0]);
-            v1 = mk(vx[i1], vy[i1], vz[i1]);
-            v2 = mk(vx[i2], vy[i2], vz[i2]);
-            float* f = reinterpret_cast<float*>(rec) + 9 * (size_t)p;
-            f[0] = v0.x; f[1] = v0.y; f[2] = v0.z;
-            f[3] = v1.x; f[4] = v1.y; f[5] = v1.z;
-            f[6] = v2.x; f[7] = v2.y; f[8] = v2.z;
-        } else {
-            load_tri(rec, p, v0, v1, v2);
-        }
-        f3 lo, hi;
-        tri_bounds(v0, v1, v2, lo, hi);
-        if (kMulti && T.object_grids) object_box_cells(lo, hi, bmin, csr, rx, ry, rz, mn, mx);
-        else box_cells(lo, hi, bmin, csr, rx, ry, rz, mn, mx);
-        cnt = (uint32_t)((mx[0] - mn[0]) * (mx[1] - mn[1]) * (mx[2] - mn[2]));
-    }
-
-    const uint32_t kcell_z = (uint32_t)rx * (uint32_t)ry;
-    if (!kExact && !kWrite) {
-        const uint32_t s = wave_sum(cnt);
-        if (lane == 0) wave_counts[wg] = s;
-        return;
-    }
-
-    WaveItems& W = sh[wl];
-    const uint32_t inc = wave_incl_scan(cnt);
-    const uint32_t total = __shfl(inc, kWave - 1, kWave);
-    W.excl[lane] = inc - cnt;
-    W.lo[0][lane] = mn[0]; W.lo[1][lane] = mn[1]; W.lo[2][lane] = mn[2];
-    W.dx[lane] = mx[0] - mn[0];
-    W.dy[lane] = mx[1] - mn[1];
-    W.id[lane] = p;
-    if (kMulti) {
-        W.gx[lane] = (uint32_t)rx;
-        W.gz[lane] = kcell_z;
-        W.cbase[lane] = cbase;
-    }
-    if (kExact) {
-        W.v[0][lane] = v0.x; W.v[1][lane] = v0.y; W.v[2][lane] = v0.z;
-        W.v[3][lane] = v1.x; W.v[4][lane] = v1.y; W.v[5][lane] = v1.z;
-        W.v[6][lane] = v2.x; W.v[7][lane] = v2.y; W.v[8][lane] = v2.z;
-        const f3 n = normalize(cross(v1 - v0, v2 - v0));
-        W.n[0][lane] = n.x; W.n[1][lane] = n.y; W.n[2][lane] = n.z;
-        const f3 half = cs * 0.505f;
-        f3 m = mk((float)mn[0], (float)mn[1], (float)mn[2]);
-        m = m * cs;
-        m = m + bmin + half;
-        W.mcc[0][lane] = m.x; W.mcc[1][lane] = m.y; W.mcc[2][lane] = m.z;
-    }
-    wave_sync();
-
-    const f3 half = cs * 0.505f;
-    const uint64_t lt = __lanemask_lt();
-    uint32_t run = kWrite ? wave_offsets[wg] : 0u;
-    for (uint32_t j0 = 0; j0 < total; j0 += kWave) {
-        const uint32_t j = j0 + (uint32_t)lane;
-        bool ok = false;
-        uint32_t key = 0, id = 0;
-        if (j < total) {
-            const int o = wave_owner(W.excl, j);
-            const uint32_t k = j - W.excl[o];
-            const uint32_t dxo = (uint32_t)W.dx[o], dyo = (uint32_t)W.dy[o];
-            const int ix = (int)(k % dxo), t = (int)(k / dxo);
-            const int iy = t % (int)dyo, iz = t / (int)dyo;
-            const int x = W.lo[0][o] + ix, y = W.lo[1][o] + iy, z = W.lo[2][o] + iz;
-            id = W.id[o];
-            if (kMulti) key = W.cbase[o] + (uint32_t)x + (uint32_t)y * W.gx[o] + (uint32_t)z * W.gz[o];
-            else key = (uint32_t)x + (uint32_t)y * (uint32_t)rx + (uint32_t)z * kcell_z;
-            if (kExact) {
-                const f3 c = mk(centre_along(W.mcc[0][o], cs.x, ix), centre_along(W.mcc[1][o], cs.y, iy),
-                                centre_along(W.mcc[2][o], cs.z, iz));
-                const f3 a = mk(W.v[0][o], W.v[1][o], W.v[2][o]);
-                const f3 b = mk(W.v[3][o], W.v[4][o], W.v[5][o]);
-                const f3 d = mk(W.v[6][o], W.v[7][o], W.v[8][o]);
-                ok = tri_cell_overlap(a, b, d, mk(W.n[0][o], W.n[1][o], W.n[2][o]), c, half);
-            } else {
-                ok = true;
+    // this wave's items: itself, or every step-th slice of the list
+    uint32_t item = own ? 0u : (blockIdx.x - own_blocks) * kWavesPerBlock + (uint32_t)wl;
+    const uint32_t step = own ? 1u : (gridDim.x - own_blocks) * kWavesPerBlock;
+    const uint32_t items = own ? 1u : st->heavy * kPairSlices;
+    for (; item < items; item += step) {
+        uint32_t wg = blockIdx.x * kWavesPerBlock + (uint32_t)wl, jb = 0, slice = 0;
+        if (!own) {
+            const uint2 e = list.waves[item / kPairSlices];
+            wg = e.x;
+            slice = item % kPairSlices;
+            jb = slice * slice_len(e.y);
+            if (jb >= e.y) {
+                if (kPass == kPairsSlices && lane == 0) list.slice_pairs[item] = 0u;
+                continue;
             }
         }
-        const uint64_t bal = __ballot(ok);
-        if (kWrite && ok) {
-            const uint32_t pos = run + (uint32_t)__popcll(bal & lt);
-            keys[pos] = key;
-            vals[pos] = id;
+        const uint32_t p = wg * kWave + lane;
+        const bool valid = p < nt;
+        const GridParams* g = gp;
+        uint32_t cbase = 0;
+        if (kMulti) {
+            const uint32_t sc = T.tri_scene[valid ? p : nt - 1u];
+            g = T.gps + sc;
+            cbase = T.cell_base[sc];
         }
-        run += (uint32_t)__popcll(bal);
+        const f3 bmin = mk(g->bmin[0], g->bmin[1], g->bmin[2]);
+        const f3 cs = mk(g->cs[0], g->cs[1], g->cs[2]);
+        const f3 csr = mk(g->csr[0], g->csr[1], g->csr[2]);
+        const int rx = g->res[0], ry = g->res[1], rz = g->res[2];
+
+        f3 v0 = rep(0.f), v1 = rep(0.f), v2 = rep(0.f);
+        uint32_t cnt = 0;
+        int mn[3] = { 0, 0, 0 }, mx[3] = { 0, 0, 0 };
+        if (valid) {
+            if (kPass == kPairsCount) {
+                const uint32_t i0 = idx[3 * (size_t)p], i1 = idx[3 * (size_t)p + 1], i2 = idx[3 * (size_t)p + 2];
+                v0 = mk(vx[i0], vy[i0], vz[i0]);
+                v1 = mk(vx[i1], vy[i1], vz[i1]);
+                v2 = mk(vx[i2], vy[i2], vz[i2]);
+                float* f = reinterpret_cast<float*>(rec) + 9 * (size_t)p;
+                f[0] = v0.x; f[1] = v0.y; f[2] = v0.z;
+                f[3] = v1.x; f[4] = v1.y; f[5] = v1.z;
+                f[6] = v2.x; f[7] = v2.y; f[8] = v2.z;
+            } else {
+                load_tri(rec, p, v0, v1, v2);
+            }
+            f3 lo, hi;
+            tri_bounds(v0, v1, v2, lo, hi);
+            if (kMulti && T.object_grids) object_box_cells(lo, hi, bmin, csr, rx, ry, rz, mn, mx);
+            else box_cells(lo, hi, bmin, csr, rx, ry, rz, mn, mx);
+            cnt = (uint32_t)((mx[0] - mn[0]) * (mx[1] - mn[1]) * (mx[2] - mn[2]));
+        }
+
+        if (!kExact && kPass == kPairsCount) {
+            const uint32_t s = wave_sum(cnt);
+            if (lane == 0) {
+                wave_counts[wg] = s;
+                if (s >= kPairsHeavy) list.waves[atomicAdd(&st->heavy, 1u)] = make_uint2(wg, s);
+            }
+            return;
+        }
+
+        const uint32_t kcell_z = (uint32_t)rx * (uint32_t)ry;
+        const uint32_t inc = wave_incl_scan(cnt);
+        const uint32_t ex = inc - cnt;
+        const uint32_t total = (uint32_t)__builtin_amdgcn_readlane((int)inc, kWave - 1);
+        if (own && total >= kPairsHeavy) {      // the list's slices do it
+            if (kPass == kPairsCount && lane == 0) {
+                wave_counts[wg] = 0u;
+                list.waves[atomicAdd(&st->heavy, 1u)] = make_uint2(wg, total);
+            }
+            return;
+        }
+        W.excl[lane] = ex;
+        W.lo[0][lane] = mn[0]; W.lo[1][lane] = mn[1]; W.lo[2][lane] = mn[2];
+        W.dx[lane] = mx[0] - mn[0];
+        W.dy[lane] = mx[1] - mn[1];
+        W.id[lane] = p;
+        if (kMulti) {
+            W.gx[lane] = (uint32_t)rx;
+            W.gz[lane] = kcell_z;
+            W.cbase[lane] = cbase;
+        }
+        if (kExact) {
+            W.v[0][lane] = v0.x; W.v[1][lane] = v0.y; W.v[2][lane] = v0.z;
+            W.v[3][lane] = v1.x; W.v[4][lane] = v1.y; W.v[5][lane] = v1.z;
+            W.v[6][lane] = v2.x; W.v[7][lane] = v2.y; W.v[8][lane] = v2.z;
+            const f3 n = normalize(cross(v1 - v0, v2 - v0));
+            W.n[0][lane] = n.x; W.n[1][lane] = n.y; W.n[2][lane] = n.z;
+            const f3 half = cs * 0.505f;
+            f3 m = mk((float)mn[0], (float)mn[1], (float)mn[2]);
+            m = m * cs;
+            m = m + bmin + half;
+            W.mcc[0][lane] = m.x; W.mcc[1][lane] = m.y; W.mcc[2][lane] = m.z;
+        }
+        wave_sync();
+
+        const f3 half = cs * 0.505f;
+        const uint64_t lt = __lanemask_lt();
+        uint32_t je = total, run = 0;
+        if (kWrite) run = wave_offsets[wg];
+        if (!own) {
+            je = total - jb < slice_len(total) ? total : jb + slice_len(total);
+            if (kWrite && kExact) {
+                // the pairs of the wave's slices before this one
+                const uint32_t c = lane < slice ? list.slice_pairs[item - slice + lane] : 0u;
+                run += wave_sum(c);
+            } else if (kWrite) {
+                run += jb;
+            }
+        }
+        const uint32_t run0 = run;
+        for (uint32_t j0 = jb; j0 < je; j0 += kWave) {
+            const uint32_t j = j0 + lane;
+            const uint32_t o = list_owner(W.mark, lane, ex, cnt, j0);
+            bool ok = false;
+            uint32_t key = 0, id = 0;
+            if (j < je) {
+                const uint32_t k = j - W.excl[o];
+                const uint32_t dxo = (uint32_t)W.dx[o], dyo = (uint32_t)W.dy[o];
+                const int ix = (int)(k % dxo), t = (int)(k / dxo);
+                const int iy = t % (int)dyo, iz = t / (int)dyo;
+                const int x = W.lo[0][o] + ix, y = W.lo[1][o] + iy, z = W.lo[2][o] + iz;
+                id = W.id[o];
+                if (kMulti) key = W.cbase[o] + (uint32_t)x + (uint32_t)y * W.gx[o] + (uint32_t)z * W.gz[o];
+                else key = (uint32_t)x + (uint32_t)y * (uint32_t)rx + (uint32_t)z * kcell_z;
+                if (kExact) {
+                    const f3 c = mk(centre_along(W.mcc[0][o], cs.x, ix), centre_along(W.mcc[1][o], cs.y, iy),
+                                    centre_along(W.mcc[2][o], cs.z, iz));
+                    const f3 a = mk(W.v[0][o], W.v[1][o], W.v[2][o]);
+                    const f3 b = mk(W.v[3][o], W.v[4][o], W.v[5][o]);
+                    const f3 d = mk(W.v[6][o], W.v[7][o], W.v[8][o]);
+                    ok = tri_cell_overlap(a, b, d, mk(W.n[0][o], W.n[1][o], W.n[2][o]), c, half);
+                } else {
+                    ok = true;
+                }
+            }
+            const uint64_t bal = __ballot(ok);
+            if (kWrite && ok) {
+                const uint32_t pos = run + (uint32_t)__popcll(bal & lt);
+                keys[pos] = key;
+                vals[pos] = id;
+            }
+            run += (uint32_t)__popcll(bal);
+        }
+        if (!kWrite && lane == 0) {
+            if (own) {
+                wave_counts[wg] = run - run0;
+            } else {
+                list.slice_pairs[item] = run - run0;
+                atomicAdd(wave_counts + wg, run - run0);
+            }
+        }
+        wave_sync();      // the next item writes the lists again
     }
-    if (!kWrite && lane == 0) wave_counts[wg] = run;
 }
 
 // prepareCellRanges (UniformGridBuildKernels.h:384-487) on sorted keys:
@@ -568,8 +666,8 @@ __global__ __launch_bounds__(kBlock) void k_leaf_pairs(
         const uint32_t j = j0 + (uint32_t)lane;
         const bool ok = j < total;
         uint32_t key = 0, id = 0;
+        const uint32_t o = list_owner(W.mark, (uint32_t)lane, inc - cnt, cnt, j0);
         if (ok) {
-            const int o = wave_owner(W.excl, j);
             const uint32_t k = j - W.excl[o];
             const uint32_t dxo = (uint32_t)W.dx[o], dyo = (uint32_t)W.dy[o];
             const uint32_t ix = k % dxo, t = k / dxo;
@@ -801,6 +899,29 @@ void launch_grid_setup(GridParams* gp, BuildStatus* st, uint32_t nprims, float l
     hipLaunchKernelGGL(k_grid_setup, dim3(1), dim3(64), 0, s, gp, st, nprims, lambda, cells_cap);
 }
 
+namespace {
+
+// workgroups beside the owners' that take the listed waves' slices: they end at
+// once where nothing is listed
+uint32_t slice_blocks(uint32_t own_blocks)
+{
+    return own_blocks / 4 < 128u ? 128u : (own_blocks / 4 > 1024u ? 1024u : own_blocks / 4);
+}
+
+PairList pair_list(uint32_t* wave_offsets, uint32_t waves_cap, uint32_t nt)
+{
+    const uint32_t waves = cdiv(nt > 0 ? nt : 1, kWave);
+    uint2* w = (uint2*)(wave_offsets + waves_cap);       // waves_cap is even
+    return PairList{ w, (uint32_t*)(w + waves) };
+}
+
+}  // namespace
+
+size_t wave_offsets_words(uint32_t waves_cap, uint32_t nt)
+{
+    return (size_t)waves_cap + (size_t)cdiv(nt > 0 ? nt : 1, kWave) * (2 + kPairSlices);
+}
+
 void run_build(const BuildArgs& a, BuildBuffers& b, hipStream_t s)
 {
     const uint32_t nt = a.nt;
@@ -813,22 +934,31 @@ void run_build(const BuildArgs& a, BuildBuffers& b, hipStream_t s)
     launch_grid_setup(b.params, st, nt, a.lambda_top, b.cells_cap, s);
 
     // ---- top level / uniform: count (and clear the cells), scan, write ----
-    if (exact)
-        hipLaunchKernelGGL((k_top_pairs<true, false>), dim3(blocks), dim3(kBlock), 0, s, a.idx, a.vx,
-                           a.vy, a.vz, nt, b.params, st, b.rec, b.wave_counts, nullptr, nullptr, nullptr, b.waves_cap,
-                           SceneTable{}, b.cells, &b.params->num_cells);
-    else
-        hipLaunchKernelGGL((k_top_pairs<false, false>), dim3(blocks), dim3(kBlock), 0, s, a.idx, a.vx,
-                           a.vy, a.vz, nt, b.params, st, b.rec, b.wave_counts, nullptr, nullptr, nullptr, b.waves_cap,
-                           SceneTable{}, b.cells, &b.params->num_cells);
+    const PairList list = pair_list(b.wave_offsets, b.waves_cap, nt);
+    const uint32_t extra = slice_blocks(blocks);
+    const SceneTable none{};
+    if (exact) {
+        hipLaunchKernelGGL((k_top_pairs<true, kPairsCount>), dim3(blocks), dim3(kBlock), 0, s, a.idx, a.vx, a.vy, a.vz,
+                           nt, b.params, st, b.rec, b.wave_counts, nullptr, nullptr, nullptr, b.waves_cap, blocks,
+                           list, none, b.cells, &b.params->num_cells);
+        hipLaunchKernelGGL((k_top_pairs<true, kPairsSlices>), dim3(extra), dim3(kBlock), 0, s, a.idx, a.vx, a.vy, a.vz,
+                           nt, b.params, st, b.rec, b.wave_counts, nullptr, nullptr, nullptr, b.waves_cap, 0u, list,
+                           none);
+    } else {
+        hipLaunchKernelGGL((k_top_pairs<false, kPairsCount>), dim3(blocks), dim3(kBlock), 0, s, a.idx, a.vx, a.vy,
+                           a.vz, nt, b.params, st, b.rec, b.wave_counts, nullptr, nullptr, nullptr, b.waves_cap, blocks,
+                           list, none, b.cells, &b.params->num_cells);
+    }
     const ScanCheck pairs_check{ st, b.pairs_cap, kOverflowPairs, &st->n_pairs_eff };
     scan_exclusive_1p(b.wave_counts, b.wave_offsets, 1, waves, nullptr, &st->num_pairs, &pairs_check, b.scan, s);
     if (exact)
-        hipLaunchKernelGGL((k_top_pairs<true, true>), dim3(blocks), dim3(kBlock), 0, s, a.idx, a.vx,
-                           a.vy, a.vz, nt, b.params, st, b.rec, nullptr, b.wave_offsets, b.keys, b.vals, b.waves_cap);
+        hipLaunchKernelGGL((k_top_pairs<true, kPairsWrite>), dim3(blocks + extra), dim3(kBlock), 0, s, a.idx, a.vx,
+                           a.vy, a.vz, nt, b.params, st, b.rec, nullptr, b.wave_offsets, b.keys, b.vals, b.waves_cap,
+                           blocks, list, none);
     else
-        hipLaunchKernelGGL((k_top_pairs<false, true>), dim3(blocks), dim3(kBlock), 0, s, a.idx, a.vx,
-                           a.vy, a.vz, nt, b.params, st, b.rec, nullptr, b.wave_offsets, b.keys, b.vals, b.waves_cap);
+        hipLaunchKernelGGL((k_top_pairs<false, kPairsWrite>), dim3(blocks + extra), dim3(kBlock), 0, s, a.idx, a.vx,
+                           a.vy, a.vz, nt, b.params, st, b.rec, nullptr, b.wave_offsets, b.keys, b.vals, b.waves_cap,
+                           blocks, list, none);
 
     // ---- sort by cell key, then cell ranges ----
     const int cell_bits = bits_for(b.cells_cap);
@@ -896,12 +1026,15 @@ void run_build_batch(const BuildArgs& a, BuildBuffers& b, const SceneTable& T, u
     hipLaunchKernelGGL(k_batch_total, dim3(1), dim3(64), 0, s, T, b.params, st, b.cells_cap);
 
     // ---- top level: count, scan, write ----
-    hipLaunchKernelGGL((k_top_pairs<false, false, true>), dim3(blocks), dim3(kBlock), 0, s, a.idx, a.vx, a.vy,
-                       a.vz, nt, b.params, st, b.rec, b.wave_counts, nullptr, nullptr, nullptr, b.waves_cap, T);
+    const PairList list = pair_list(b.wave_offsets, b.waves_cap, nt);
+    hipLaunchKernelGGL((k_top_pairs<false, kPairsCount, true>), dim3(blocks), dim3(kBlock), 0, s, a.idx, a.vx, a.vy,
+                       a.vz, nt, b.params, st, b.rec, b.wave_counts, nullptr, nullptr, nullptr, b.waves_cap, blocks,
+                       list, T);
     const ScanCheck pairs_check{ st, b.pairs_cap, kOverflowPairs, &st->n_pairs_eff };
     scan_exclusive_1p(b.wave_counts, b.wave_offsets, 1, waves, nullptr, &st->num_pairs, &pairs_check, b.scan, s);
-    hipLaunchKernelGGL((k_top_pairs<false, true, true>), dim3(blocks), dim3(kBlock), 0, s, a.idx, a.vx, a.vy,
-                       a.vz, nt, b.params, st, b.rec, nullptr, b.wave_offsets, b.keys, b.vals, b.waves_cap, T);
+    hipLaunchKernelGGL((k_top_pairs<false, kPairsWrite, true>), dim3(blocks + slice_blocks(blocks)), dim3(kBlock), 0,
+                       s, a.idx, a.vx, a.vy, a.vz, nt, b.params, st, b.rec, nullptr, b.wave_offsets, b.keys, b.vals,
+                       b.waves_cap, blocks, list, T);
 
     // ---- sort by global cell key, cell ranges ----
     radix_sort_pairs(b.keys, b.vals, b.keys_sorted, b.top_vals_sorted, b.pairs_cap, &st->n_pairs_eff,
@@ -1283,13 +1416,15 @@ void run_build_hier(const HierArgs& a, HierBuffers& b, hipStream_t s)
     T.object_grids = 1;
     const uint32_t waves = cdiv(nt > 0 ? nt : 1, kWave);
     const uint32_t blocks = cdiv(waves, kWavesPerBlock);
-    hipLaunchKernelGGL((k_top_pairs<false, false, true>), dim3(blocks), dim3(kBlock), 0, s, a.idx, a.vx, a.vy, a.vz,
-                       nt, b.top, st, b.rec, b.wave_counts, nullptr, nullptr, nullptr, b.waves_cap, T, b.obj_cells,
-                       &st->n_leaves_eff);
+    const PairList list = pair_list(b.wave_offsets, b.waves_cap, nt);
+    hipLaunchKernelGGL((k_top_pairs<false, kPairsCount, true>), dim3(blocks), dim3(kBlock), 0, s, a.idx, a.vx, a.vy,
+                       a.vz, nt, b.top, st, b.rec, b.wave_counts, nullptr, nullptr, nullptr, b.waves_cap, blocks, list,
+                       T, b.obj_cells, &st->n_leaves_eff);
     const ScanCheck refs_check{ st, b.leaf_pairs_cap, kOverflowLeafPairs, &st->n_leaf_pairs_eff };
     scan_exclusive_1p(b.wave_counts, b.wave_offsets, 1, waves, nullptr, &st->num_leaf_pairs, &refs_check, b.scan, s);
-    hipLaunchKernelGGL((k_top_pairs<false, true, true>), dim3(blocks), dim3(kBlock), 0, s, a.idx, a.vx, a.vy, a.vz,
-                       nt, b.top, st, b.rec, nullptr, b.wave_offsets, b.keys, b.vals, b.waves_cap, T);
+    hipLaunchKernelGGL((k_top_pairs<false, kPairsWrite, true>), dim3(blocks + slice_blocks(blocks)), dim3(kBlock), 0,
+                       s, a.idx, a.vx, a.vy, a.vz, nt, b.top, st, b.rec, nullptr, b.wave_offsets, b.keys, b.vals,
+                       b.waves_cap, blocks, list, T);
     radix_sort_pairs(b.keys, b.vals, b.keys_sorted, b.prims, b.leaf_pairs_cap, &st->n_leaf_pairs_eff,
                      bits_for(b.leaves_cap), b.sort, s);
     hipLaunchKernelGGL(k_ranges, dim3(range_blocks(b.leaf_pairs_cap)), dim3(256), 0, s, b.keys_sorted,

@@ -35,7 +35,8 @@ struct BuildStatus {
     uint32_t n_pairs_eff;       // sizes the later kernels use: 0 after an overflow
     uint32_t n_leaves_eff;
     uint32_t n_leaf_pairs_eff;
-    uint32_t pad[2];
+    uint32_t heavy;             // waves of triangles with many candidates, listed for the pair passes
+    uint32_t pad;
 };
 
 // The per-frame selection of a captured frame (HIP graph): key frames, the
@@ -146,16 +147,6 @@ __device__ __forceinline__ float wave_max(float v)
 #pragma unroll
     for (int d = kWave / 2; d >= 1; d >>= 1) v = fmaxf(v, __shfl_xor(v, d, kWave));
     return v;
-}
-
-// largest o in [0, 64) with excl[o] <= j (excl[0] == 0 <= j)
-__device__ __forceinline__ int wave_owner(const uint32_t* excl, uint32_t j)
-{
-    int o = 0;
-#pragma unroll
-    for (int step = 32; step >= 1; step >>= 1)
-        if (excl[o + step] <= j) o += step;
-    return o;
 }
 
 // triangle record: nine packed floats (v0, v1, v2) per triangle, in a float4

@@ -326,7 +326,7 @@ hr_status reserve_build(hr_ctx* c)
     const uint32_t waves = cdiv(std::max<uint64_t>(std::max(nt, c->pairs_cap), 1), 64);
     const uint32_t waves_cap = (waves + 3) / 4 * 4 + 4;
     HR_TRY(c->wave_counts.reserve(waves_cap));
-    HR_TRY(c->wave_offsets.reserve(waves_cap));
+    HR_TRY(c->wave_offsets.reserve(hr::wave_offsets_words((uint32_t)c->wave_counts.cap, nt)));
     HR_TRY(c->keys.reserve(pair_max));
     HR_TRY(c->vals.reserve(pair_max));
     HR_TRY(c->keys_sorted.reserve(pair_max));
