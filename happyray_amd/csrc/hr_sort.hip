@@ -204,32 +204,54 @@ __global__ void k_fill(uint32_t* __restrict__ p, uint32_t value, size_t n_cap,
 // radix sort
 // ---------------------------------------------------------------------------
 
-constexpr int kRadix = 256;
-constexpr int kSortItems = kSortTile / kBlock;   // 8
-constexpr int kSortWaves = kBlock / kWave;       // 4
-
 // Chunked LSD radix sort.  A pass runs over a fixed grid of G workgroups;
 // workgroup b owns a contiguous chunk of whole 2048-key tiles.
 //  1. k_sort_count: each workgroup counts the digits of its chunk (one LDS
-//     histogram per wave; counts do not depend on the order of the adds)
-//     into counts[digit * G + b];
-//  2. k_sort_rowscan: one workgroup per digit scans that digit's row (each
+//     histogram per wave; counts do not depend on the order of the adds);
+//  2. k_sort_rowscan: one workgroup per digit scans that digit's counts (each
 //     chunk's first slot among the digit's keys) and writes the digit total;
 //  3. k_sort_scatter: each workgroup adds the totals of the smaller digits to
-//     its row entries, then walks its tiles in order, ranks the keys
-//     of a tile by digit (stable), stages the tile in LDS by digit and writes
-//     each digit's run at the chunk's running offset.
+//     its own, then walks its tiles in order, ranks the keys of a tile by
+//     digit (stable), stages the tile in LDS by digit and writes each digit's
+//     run at the chunk's running offset.
 // Every chunk's tiles keep their order, so the sort is stable.
+//
+// Up to kSortFold workgroups there is no step 2: every scatter workgroup adds
+// up the chunks' counts itself, read a whole row of digits at a time.  That
+// reads G^2 rows in all, little at this size, and saves a launch.
 
 constexpr int kSortGrid = 1024;                  // workgroups per pass (at most)
+constexpr uint32_t kSortFold = 128;
+
+// The scatter has 1024 threads of two keys each: its time on few tiles is the
+// latency of a tile's steps (ranks of a wave's keys one after the other), and
+// on many tiles four workgroups of 256 per CU left the CU half empty.
+constexpr int kScatterBlock = 1024;
+constexpr int kScatterItems = kSortTile / kScatterBlock;   // 2
+constexpr int kScatterWaves = kScatterBlock / kWave;       // 16
+
+template <int kWaves>
+__device__ __forceinline__ uint32_t waves_excl_scan(uint32_t v, uint32_t* lds_waves)
+{
+    const uint32_t w = threadIdx.x / kWave;
+    const uint32_t inc = wave_incl_scan(v);
+    if (__lane_id() == kWave - 1) lds_waves[w] = inc;
+    __syncthreads();
+    uint32_t off = 0;
+#pragma unroll
+    for (uint32_t i = 0; i < (uint32_t)kWaves; ++i) off += i < w ? lds_waves[i] : 0u;
+    __syncthreads();
+    return off + inc - v;
+}
 
 // rank of each of the wave's keys among the equal digits of the wave (lanes
 // in order), and the wave's counts per digit accumulated into h[digit]
-__device__ __forceinline__ uint32_t wave_digit_rank(uint32_t d, bool valid, uint32_t* h)
+template <int kBits>
+__device__ __forceinline__ uint32_t wave_digit_rank(uint32_t d, bool valid, uint16_t* h)
 {
     uint64_t match = __ballot(valid);
 #pragma unroll
-    for (int b = 0; b < 8; ++b) {
+    for (int b = 0; b < kBits; ++b) {
         const bool bit = (d >> b) & 1u;
         const uint64_t bal = __ballot(bit);
         match &= bit ? bal : ~bal;
@@ -237,7 +259,7 @@ __device__ __forceinline__ uint32_t wave_digit_rank(uint32_t d, bool valid, uint
     const uint32_t below = (uint32_t)__popcll(match & __lanemask_lt());
     const uint32_t cnt = h[d];
     wave_sync();
-    if (valid && below == 0u) h[d] = cnt + (uint32_t)__popcll(match);
+    if (valid && below == 0u) h[d] = (uint16_t)(cnt + (uint32_t)__popcll(match));
     wave_sync();
     return cnt + below;
 }
@@ -251,40 +273,49 @@ __device__ __forceinline__ void chunk_tiles(uint32_t n, uint32_t b, uint32_t g, 
     if (t0 > t1) t0 = t1;
 }
 
+// counts: digit-major (row d: the chunks' counts of digit d) for the row scan,
+// chunk-major where the scatter adds them up (kFold)
+template <int kBits, bool kFold>
 __global__ __launch_bounds__(kBlock) void k_sort_count(const uint32_t* __restrict__ keys,
                                                        const uint32_t* __restrict__ n_dev, int shift,
                                                        uint32_t* __restrict__ counts)
 {
-    __shared__ uint32_t h[kSortWaves][kRadix];
+    constexpr uint32_t kRadix = 1u << kBits;
+    constexpr int kWaves = kBlock / kWave;
+    constexpr int kItems = kSortTile / kBlock;
+    __shared__ uint32_t h[kWaves][kRadix];
     const int w = (int)threadIdx.x / kWave;
     const int lane = (int)__lane_id();
+    for (uint32_t d = threadIdx.x; d < kRadix; d += kBlock)
 #pragma unroll
-    for (int i = 0; i < kSortWaves; ++i) h[i][threadIdx.x] = 0u;
-    __syncthreads();
+        for (int i = 0; i < kWaves; ++i) h[i][d] = 0u;
     const uint32_t n = *n_dev;
     uint32_t t0, t1;
     chunk_tiles(n, blockIdx.x, gridDim.x, t0, t1);
+    if (kFold && t0 >= t1) return;      // the scatter reads the chunks that have tiles
+    __syncthreads();
     for (uint32_t t = t0; t < t1; ++t) {
-        const uint32_t base = t * kSortTile + (uint32_t)w * (kWave * kSortItems) + lane;
-        uint32_t kr[kSortItems];
+        const uint32_t base = t * kSortTile + (uint32_t)w * (kWave * kItems) + lane;
+        uint32_t kr[kItems];
 #pragma unroll
-        for (int k = 0; k < kSortItems; ++k) {
+        for (int k = 0; k < kItems; ++k) {
             const uint32_t i = base + (uint32_t)k * kWave;
             kr[k] = i < n ? keys[i] : 0u;
         }
 #pragma unroll
-        for (int k = 0; k < kSortItems; ++k) {
+        for (int k = 0; k < kItems; ++k) {
             const uint32_t i = base + (uint32_t)k * kWave;
             if (i < n) atomicAdd(&h[w][(kr[k] >> shift) & (kRadix - 1)], 1u);
         }
     }
     __syncthreads();
-    uint32_t c = 0;
+    for (uint32_t d = threadIdx.x; d < kRadix; d += kBlock) {
+        uint32_t c = 0;
 #pragma unroll
-    for (int i = 0; i < kSortWaves; ++i) c += h[i][threadIdx.x];
-    // digit-major: the exclusive scan of this array is each chunk's first
-    // output position per digit
-    counts[(size_t)threadIdx.x * gridDim.x + blockIdx.x] = c;
+        for (int i = 0; i < kWaves; ++i) c += h[i][d];
+        if (kFold) counts[(size_t)blockIdx.x * kRadix + d] = c;
+        else counts[(size_t)d * gridDim.x + blockIdx.x] = c;
+    }
 }
 
 // one workgroup per digit d: the exclusive scan of counts[d * G .. d * G + G)
@@ -293,7 +324,7 @@ __global__ __launch_bounds__(kBlock) void k_sort_count(const uint32_t* __restric
 __global__ __launch_bounds__(kBlock) void k_sort_rowscan(uint32_t* __restrict__ counts, uint32_t g,
                                                          uint32_t* __restrict__ totals)
 {
-    __shared__ uint32_t lds_scan[kSortWaves];
+    __shared__ uint32_t lds_scan[kBlock / kWave];
     constexpr uint32_t kPer = (uint32_t)kSortGrid / kBlock;
     uint32_t* row = counts + (size_t)blockIdx.x * g;
     uint32_t v[kPer];
@@ -315,85 +346,136 @@ __global__ __launch_bounds__(kBlock) void k_sort_rowscan(uint32_t* __restrict__ 
     if (threadIdx.x == 0) totals[blockIdx.x] = all;
 }
 
-__global__ __launch_bounds__(kBlock) void k_sort_scatter(
+template <int kBits, bool kFold>
+__global__ __launch_bounds__(kScatterBlock) void k_sort_scatter(
     const uint32_t* __restrict__ keys_src, const uint32_t* __restrict__ vals_src,
     uint32_t* __restrict__ keys_dst, uint32_t* __restrict__ vals_dst,
     const uint32_t* __restrict__ n_dev, int shift, const uint32_t* __restrict__ counts,
     const uint32_t* __restrict__ totals)
 {
+    constexpr uint32_t kRadix = 1u << kBits;
     __shared__ uint32_t skeys[kSortTile];
     __shared__ uint32_t svals[kSortTile];
-    __shared__ uint32_t whist[kSortWaves][kRadix];
+    __shared__ uint32_t whist2[kScatterWaves * kRadix / 2];    // 16-bit counts: a tile has 2048 keys
     __shared__ uint32_t dstart[kRadix];
     __shared__ uint32_t offs[kRadix];
-    __shared__ uint32_t lds_scan[kSortWaves];
+    __shared__ uint32_t lds_scan[kScatterWaves];
+    uint16_t* whist = (uint16_t*)whist2;
 
     const uint32_t n = *n_dev;
     uint32_t t0, t1;
     chunk_tiles(n, blockIdx.x, gridDim.x, t0, t1);
     if (t0 >= t1) return;
-    const int w = (int)threadIdx.x / kWave;
-    const int lane = (int)__lane_id();
+    const uint32_t w = threadIdx.x / kWave;
+    const uint32_t lane = __lane_id();
+    const uint32_t d = threadIdx.x;       // this thread's digit, where there is one
+    const bool has_d = d < kRadix;
+    uint16_t* wh = whist + w * kRadix;
+    uint32_t kr[kScatterItems], vr[kScatterItems];
+    auto load = [&](uint32_t t) {
+#pragma unroll
+        for (int k = 0; k < kScatterItems; ++k) {
+            const uint32_t i = t * kSortTile + w * (kWave * kScatterItems) + (uint32_t)k * kWave + lane;
+            kr[k] = i < n ? keys_src[i] : 0u;
+            vr[k] = i < n ? vals_src[i] : 0u;
+        }
+    };
+    load(t0);
     {
+        uint32_t total = 0, before = 0;   // of the digit: all keys, those of the earlier chunks
+        if (kFold) {
+            // one tile per chunk here; the threads share the rows of a digit
+            constexpr uint32_t kShare = kScatterBlock / kRadix;
+            const uint32_t chunks = (n + kSortTile - 1) / kSortTile;
+            const uint32_t dd = threadIdx.x % kRadix, q = threadIdx.x / kRadix;
+#pragma unroll 8
+            for (uint32_t b = q; b < chunks; b += kShare) {
+                const uint32_t c = counts[(size_t)b * kRadix + dd];
+                total += c;
+                before += b < blockIdx.x ? c : 0u;
+            }
+            if (kShare > 1) {
+                if (q > 0) {
+                    skeys[(q - 1) * kRadix + dd] = total;
+                    svals[(q - 1) * kRadix + dd] = before;
+                }
+                __syncthreads();
+                if (q == 0)
+#pragma unroll
+                    for (uint32_t k = 0; k + 1 < kShare; ++k) {
+                        total += skeys[k * kRadix + dd];
+                        before += svals[k * kRadix + dd];
+                    }
+                else
+                    total = 0;
+            }
+        } else if (has_d) {
+            total = totals[d];
+            before = counts[(size_t)d * gridDim.x + blockIdx.x];
+        }
         // the digit's first slot: the keys of all smaller digits
-        uint32_t all;
-        const uint32_t base = block_excl_scan(totals[threadIdx.x], lds_scan, all);
-        offs[threadIdx.x] = base + counts[(size_t)threadIdx.x * gridDim.x + blockIdx.x];
+        const uint32_t base = waves_excl_scan<kScatterWaves>(total, lds_scan);
+        if (has_d) offs[d] = base + before;
     }
     for (uint32_t t = t0; t < t1; ++t) {
         const uint32_t base = t * kSortTile;
 #pragma unroll
-        for (int i = 0; i < kSortWaves; ++i) whist[i][threadIdx.x] = 0u;
+        for (uint32_t i = threadIdx.x; i < kScatterWaves * kRadix / 2; i += kScatterBlock) whist2[i] = 0u;
         __syncthreads();
-        uint32_t kr[kSortItems], vr[kSortItems], rank[kSortItems];
+        uint32_t rank[kScatterItems];
 #pragma unroll
-        for (int k = 0; k < kSortItems; ++k) {
-            const uint32_t i = base + (uint32_t)w * (kWave * kSortItems) + (uint32_t)k * kWave + lane;
-            const bool valid = i < n;
-            kr[k] = valid ? keys_src[i] : 0u;
-            vr[k] = valid ? vals_src[i] : 0u;
-            rank[k] = wave_digit_rank((kr[k] >> shift) & (kRadix - 1), valid, whist[w]);
+        for (int k = 0; k < kScatterItems; ++k) {
+            const uint32_t i = base + w * (kWave * kScatterItems) + (uint32_t)k * kWave + lane;
+            rank[k] = wave_digit_rank<kBits>((kr[k] >> shift) & (kRadix - 1), i < n, wh);
         }
         __syncthreads();
         {
             // per digit: prefix over the waves and the tile's digit starts
-            const uint32_t d = threadIdx.x;
             uint32_t tot = 0;
+            if (has_d) {
+                uint32_t c[kScatterWaves];
 #pragma unroll
-            for (int i = 0; i < kSortWaves; ++i) {
-                const uint32_t c = whist[i][d];
-                whist[i][d] = tot;
-                tot += c;
+                for (int i = 0; i < kScatterWaves; ++i) c[i] = whist[(uint32_t)i * kRadix + d];
+#pragma unroll
+                for (int i = 0; i < kScatterWaves; ++i) {
+                    whist[(uint32_t)i * kRadix + d] = (uint16_t)tot;
+                    tot += c[i];
+                }
             }
-            uint32_t all;
-            dstart[d] = block_excl_scan(tot, lds_scan, all);
+            const uint32_t ds = waves_excl_scan<kScatterWaves>(tot, lds_scan);
+            if (has_d) dstart[d] = ds;
         }
         __syncthreads();
 #pragma unroll
-        for (int k = 0; k < kSortItems; ++k) {
-            const uint32_t i = base + (uint32_t)w * (kWave * kSortItems) + (uint32_t)k * kWave + lane;
+        for (int k = 0; k < kScatterItems; ++k) {
+            const uint32_t i = base + w * (kWave * kScatterItems) + (uint32_t)k * kWave + lane;
             if (i < n) {
-                const uint32_t d = (kr[k] >> shift) & (kRadix - 1);
-                const uint32_t pos = dstart[d] + whist[w][d] + rank[k];
+                const uint32_t dk = (kr[k] >> shift) & (kRadix - 1);
+                const uint32_t pos = dstart[dk] + wh[dk] + rank[k];
                 skeys[pos] = kr[k];
                 svals[pos] = vr[k];
             }
         }
+        if (t + 1 < t1) load(t + 1);      // in flight while this tile is written
         __syncthreads();
         const uint32_t tile_n = (n - base) < kSortTile ? (n - base) : kSortTile;
-        for (uint32_t i = threadIdx.x; i < tile_n; i += kBlock) {
-            const uint32_t key = skeys[i];
-            const uint32_t d = (key >> shift) & (kRadix - 1);
-            const uint32_t dst = offs[d] + (i - dstart[d]);
-            if (dst < n) {   // always true when the counts agree; keeps a bad count in bounds
-                keys_dst[dst] = key;
-                vals_dst[dst] = svals[i];
+#pragma unroll
+        for (int k = 0; k < kScatterItems; ++k) {
+            const uint32_t i = threadIdx.x + (uint32_t)k * kScatterBlock;
+            if (i < tile_n) {
+                const uint32_t key = skeys[i];
+                const uint32_t dk = (key >> shift) & (kRadix - 1);
+                const uint32_t dst = offs[dk] + (i - dstart[dk]);
+                if (dst < n) {   // always true when the counts agree; keeps a bad count in bounds
+                    keys_dst[dst] = key;
+                    vals_dst[dst] = svals[i];
+                }
             }
         }
+        if (t + 1 >= t1) break;
         __syncthreads();
         // advance the chunk's offsets by this tile's digit counts
-        {
-            const uint32_t d = threadIdx.x;
+        if (has_d) {
             const uint32_t next = d + 1 < kRadix ? dstart[d + 1] : tile_n;
             offs[d] += next - dstart[d];
         }
@@ -433,20 +515,47 @@ static uint32_t sort_grid(uint32_t n_cap)
     return tiles < (uint32_t)kSortGrid ? tiles : (uint32_t)kSortGrid;
 }
 
-size_t sort_hist_words(uint32_t n_cap) { return 2 * (size_t)kRadix * sort_grid(n_cap); }
+constexpr int kSortMaxBits = 10;
 
-size_t sort_chain_words(uint32_t n_cap) { return scan_chain_words((uint32_t)kRadix * sort_grid(n_cap)); }
+// counts of every chunk and digit, and the digits' totals
+size_t sort_hist_words(uint32_t n_cap) { return ((size_t)1 << kSortMaxBits) * (sort_grid(n_cap) + 1u); }
+
+size_t sort_chain_words(uint32_t n_cap) { return scan_chain_words(256u * sort_grid(n_cap)); }
+
+namespace {
+
+template <int kBits>
+void sort_pass(const uint32_t* ks, const uint32_t* vs, uint32_t* kd, uint32_t* vd, uint32_t g, const uint32_t* n_dev,
+               int shift, uint32_t* hist, hipStream_t s)
+{
+    constexpr uint32_t kRadix = 1u << kBits;
+    if (g <= kSortFold) {
+        hipLaunchKernelGGL((k_sort_count<kBits, true>), dim3(g), dim3(kBlock), 0, s, ks, n_dev, shift, hist);
+        hipLaunchKernelGGL((k_sort_scatter<kBits, true>), dim3(g), dim3(kScatterBlock), 0, s, ks, vs, kd, vd, n_dev,
+                           shift, hist, nullptr);
+        return;
+    }
+    uint32_t* totals = hist + (size_t)kRadix * g;
+    hipLaunchKernelGGL((k_sort_count<kBits, false>), dim3(g), dim3(kBlock), 0, s, ks, n_dev, shift, hist);
+    hipLaunchKernelGGL(k_sort_rowscan, dim3(kRadix), dim3(kBlock), 0, s, hist, g, totals);
+    hipLaunchKernelGGL((k_sort_scatter<kBits, false>), dim3(g), dim3(kScatterBlock), 0, s, ks, vs, kd, vd, n_dev,
+                       shift, hist, totals);
+}
+
+}  // namespace
 
 void radix_sort_pairs(uint32_t* keys_in, uint32_t* vals_in, uint32_t* keys_out, uint32_t* vals_out,
                       uint32_t n_cap, const uint32_t* n_dev, int bits, SortTemp& tmp, hipStream_t s)
 {
     const uint32_t g = sort_grid(n_cap);
-    const uint32_t m = (uint32_t)kRadix * g;
-    uint32_t* counts = tmp.hist;
-    uint32_t* totals = tmp.hist + m;     // kRadix words of the second half
-    int passes = (bits + 7) / 8;
-    if (passes < 1) passes = 1;
-    if (passes > 4) passes = 4;
+    // digits of 8 bits, or of 9 or 10 where that saves a pass
+    if (bits < 1) bits = 1;
+    if (bits > 32) bits = 32;
+    int passes = (bits + 7) / 8, width = 8;
+    if ((bits + kSortMaxBits - 1) / kSortMaxBits < passes) {
+        passes = (bits + kSortMaxBits - 1) / kSortMaxBits;
+        width = (bits + passes - 1) / passes;
+    }
     uint32_t* ks = keys_in;
     uint32_t* vs = vals_in;
     for (int p = 0; p < passes; ++p) {
@@ -455,10 +564,9 @@ void radix_sort_pairs(uint32_t* keys_in, uint32_t* vals_in, uint32_t* keys_out, 
         if (p == passes - 1) { kd = keys_out; vd = vals_out; }
         else if ((p & 1) == 0) { kd = tmp.keys_tmp; vd = tmp.vals_tmp; }
         else { kd = keys_in; vd = vals_in; }
-        hipLaunchKernelGGL(k_sort_count, dim3(g), dim3(kBlock), 0, s, ks, n_dev, 8 * p, counts);
-        hipLaunchKernelGGL(k_sort_rowscan, dim3(kRadix), dim3(kBlock), 0, s, counts, g, totals);
-        hipLaunchKernelGGL(k_sort_scatter, dim3(g), dim3(kBlock), 0, s, ks, vs, kd, vd, n_dev, 8 * p, counts,
-                           totals);
+        if (width <= 8) sort_pass<8>(ks, vs, kd, vd, g, n_dev, 8 * p, tmp.hist, s);
+        else if (width == 9) sort_pass<9>(ks, vs, kd, vd, g, n_dev, 9 * p, tmp.hist, s);
+        else sort_pass<10>(ks, vs, kd, vd, g, n_dev, 10 * p, tmp.hist, s);
         ks = kd;
         vs = vd;
     }

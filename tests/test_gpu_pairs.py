@@ -53,3 +53,16 @@ def test_large_triangles_in_a_batch():
         np.testing.assert_array_equal(leaves, og.leaves())
         np.testing.assert_array_equal(prims, og.prims())
     b.close()
+
+
+# triangles and density such that the cell or leaf keys have 16, 17, 19, 20 and
+# 21 bits (digits of 8, 9 and 10) over few sort chunks and over more than 128
+@pytest.mark.parametrize("kind,tris,density", [
+    (GRID_TWO_LEVEL, 3000, 0.25), (GRID_TWO_LEVEL, 12000, 0.25), (GRID_TWO_LEVEL, 40000, 0.25),
+    (GRID_TWO_LEVEL, 100000, 0.25), (GRID_TWO_LEVEL, 140000, 1.2), (GRID_UNIFORM, 20000, 20.0),
+    (GRID_UNIFORM, 70000, 1.5), (GRID_UNIFORM, 1, 1.0), (GRID_UNIFORM, 681, 3.0)])
+def test_sort_widths(kind, tris, density):
+    sc = scenes.random_soup(tris, tris, extent=10.0, size=0.1)
+    e = gpu_engine(sc, kind, density, 2.0)
+    assert_grid_equal(e, oracle_grid(sc, kind, density, 2.0))
+    e.close()
