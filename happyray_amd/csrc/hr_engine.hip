@@ -1001,7 +1001,7 @@ hr_status enqueue_render(hr_ctx* c, hr_mode mode, int image_id, const hr_render_
         hr::launch_simple_shade(S, ra, npix, c->hits.p, c->hit_prims.p, fb, c->stream);
     } else {
         hr::launch_path_multi(S, c->cam, ra, c->hits.p, c->hit_prims.p, sh, path_buffers(c), fb,
-                              rays, c->stream, e_p2);
+                              rays, c->stream, (uint32_t)c->tuning.advance_steps, e_p2);
     }
     if (e_r1) HR_HIP(hipEventRecord(e_r1, c->stream));
     HR_HIP(hipGetLastError());

@@ -140,10 +140,12 @@ struct PathBuffers {
 };
 constexpr int kPathMaxBounces = 8;   // RFRACTION_PATH_MAX_DEPTH (PathTracer.h:23)
 // tracePath, shadow rays, computeDirectIllumination and addIndirectIllumination;
-// hits / hit_prims hold the primary hits
+// hits / hit_prims hold the primary hits; up to steps_max grid steps per lane
+// and batch of candidate tests
 void launch_path_multi(const TraceScene& S, const CameraDev& cam, const RenderArgs& ra, const float* hits,
                        const uint32_t* hit_prims, const Shading& sh, const PathBuffers& pb, float* fb,
-                       unsigned long long* ray_count, hipStream_t s, hipEvent_t after_trace = nullptr);
+                       unsigned long long* ray_count, hipStream_t s, uint32_t steps_max,
+                       hipEvent_t after_trace = nullptr);
 // fs != nullptr: a and b are blocks fs->k1 and fs->k2 of keys, chosen on the device
 void launch_frame_normals(const float* a, const float* b, uint32_t nn, float4* out, hipStream_t s,
                           const FrameSel* fs = nullptr, const float* keys = nullptr);

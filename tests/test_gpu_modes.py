@@ -77,6 +77,26 @@ def test_path_multi_parity(kind, lt, ll):
     e.close()
 
 
+@pytest.mark.parametrize("kind", [GRID_UNIFORM_EXACT, GRID_TWO_LEVEL])
+@pytest.mark.parametrize("res", [(1, 1), (7, 9), (65, 3), (51, 21)])
+def test_path_multi_ragged_images(kind, res):
+    """Images whose last wave and workgroup are partly or nearly empty."""
+    sc = mixed_cluster()
+    e = gpu_engine(sc, kind, 1.0, 3.0)
+    e.set_lights(sc.lights)
+    og = oracle_grid(sc, kind, 1.0, 3.0)
+    c = dict(sc.camera, res=res)
+    e.set_camera_dict(c)
+    cam = O.camera(c["pos"], c["dir"], c["up"], c["fov"], *res)
+    fb_o, state = None, None
+    for image in range(2):
+        fb_g = e.render_frame(image, MODE_PATH_MULTI)
+        fb_o, state, _, _, _, _ = O.render_pt_multi(og, cam, O.params(seed=SEED, nthreads=8), sc.materials,
+                                                    sc.mat_idx, sc.lights, image_id=image, fb=fb_o, state=state)
+        np.testing.assert_array_equal(fb_g, fb_o)
+    e.close()
+
+
 def test_path_multi_without_lights_leaves_the_frame():
     sc = scenes.small_box()
     e = gpu_engine(sc, GRID_TWO_LEVEL, 1.2, 2.2)
