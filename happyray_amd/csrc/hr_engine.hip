@@ -2294,7 +2294,13 @@ hr_status hr_set_instances(hr_ctx* c, const uint32_t* obj_first, uint32_t nobj, 
             d.it[k] = a.m[k][3];
         }
         d.object = a.object;
-        d.pad = 0;
+        bool in_range = true;
+        for (int r = 0; r < 3; ++r)
+            for (int k = 0; k < 3; ++k) {
+                const float v = std::fabs(a.m[r][k]);
+                in_range = in_range && (v == 0.f || (v >= 0x1p-60f && v <= 0x1p60f));
+            }
+        d.short_div = in_range ? 1u : 0u;
     }
     const uint32_t ntri = obj_first[nobj];
     std::vector<uint32_t> tri_obj(std::max(ntri, 1u), 0u);

@@ -24,7 +24,7 @@ struct InstanceDev {
     float bmin[3], bmax[3];
     float irot0[3], irot1[3], irot2[3], it[3];
     uint32_t object;
-    uint32_t pad;
+    uint32_t short_div;             // 1: every entry of irot0..2 is 0 or in [2^-60, 2^60] in magnitude
 };
 
 // Per instance: its object's grid and first object cell, gathered by the

@@ -439,32 +439,50 @@ __global__ __launch_bounds__(kBlock) void k_ao_shade_hier(HierScene H, RenderArg
 // occlusion bit is the one-ray-per-lane kernel's.
 // ---------------------------------------------------------------------------
 
+// A ray remembers the instances it has visited (see Mailbox) in eight words of
+// LDS, [id & 7][lane]: no select chains over eight registers.
+typedef uint32_t LdsMailbox[8][kWave];
+
+// grid steps that a lane takes per iteration: in an object until it has
+// candidates, in the top grid until it meets an instance
+constexpr uint32_t kObjSteps = 2, kTopSteps = 2;
+// lanes outside the objects wait until this many of the wave do (or none has
+// other work), then all take the step into an object together
+constexpr uint32_t kEnterMin = 32;
+
+// Grid steps are counted down to the side the ray leaves by (1: the last cell)
+// and the cell index runs along, so a step is three selects and no multiply.
+// A count above the resolution is a cell before the grid's near side: empty.
 struct HierRay {
     f3 org, rcp;
     float t, tterm;
     float tstop;                 // an accepted hit closer than this finishes the ray
     uint32_t best, inst;
-    Mailbox mb;
-    int cx, cy, cz;              // top grid
+    uint32_t cx, cy, cz, cell;   // top grid
     float tx, ty, tz;
     uint32_t it, end;            // instance references of the current top cell
     bool in_inst;                // an instance's object grid is being stepped
-    uint32_t ii, base, hit;
+    uint32_t ii, hit;
     float te1, tx1, rayT;
-    f3 ot, rt, dt;               // object-space origin, reciprocal direction, direction
-    f3 ocs;                      // object cell size
-    int rx, ry, rz;
-    int ocx, ocy, ocz;
+    f3 ot, dt;                   // object-space origin, direction
+    f3 od;                       // distance along the ray between object cell planes
+    uint32_t rx, ry, rz;
+    int sx, sy, sz;              // the object cell index's step along each axis
+    uint32_t ocx, ocy, ocz, ocell;
     float otx, oty, otz;
     uint32_t pit, pend;          // triangle references of the current object cell
 };
 
+__device__ __forceinline__ uint32_t steps_left(bool forward, int res, int c)
+{
+    return forward ? (uint32_t)res - (uint32_t)c : (uint32_t)c + 1u;
+}
+
 __device__ __forceinline__ void hp_top_cell(const HierScene& H, const GridRegs& G, HierRay& r)
 {
     r.it = r.end = 0u;
-    if (r.cx < G.rx && r.cx > -1 && r.cy < G.ry && r.cy > -1 && r.cz < G.rz && r.cz > -1) {
-        const uint2 cell =
-            H.top_cells[(uint32_t)r.cx + (uint32_t)r.cy * (uint32_t)G.rx + (uint32_t)r.cz * ((uint32_t)G.rx * (uint32_t)G.ry)];
+    if (r.cx <= (uint32_t)G.rx && r.cy <= (uint32_t)G.ry && r.cz <= (uint32_t)G.rz) {
+        const uint2 cell = H.top_cells[r.cell];
         r.it = cell.x;
         r.end = cell.y;
     }
@@ -473,23 +491,22 @@ __device__ __forceinline__ void hp_top_cell(const HierScene& H, const GridRegs& 
 __device__ __forceinline__ void hp_obj_cell(const HierScene& H, HierRay& r)
 {
     r.pit = r.pend = 0u;
-    if (r.ocx < r.rx && r.ocx > -1 && r.ocy < r.ry && r.ocy > -1 && r.ocz < r.rz && r.ocz > -1) {
-        const uint2 cell = H.obj_cells[r.base + (uint32_t)r.ocx + (uint32_t)r.ocy * (uint32_t)r.rx +
-                                       (uint32_t)r.ocz * ((uint32_t)r.rx * (uint32_t)r.ry)];
+    if (r.ocx <= r.rx && r.ocy <= r.ry && r.ocz <= r.rz) {
+        const uint2 cell = H.obj_cells[r.ocell];
         r.pit = cell.x;
         r.pend = cell.y;
     }
 }
 
 // set up the top-grid DDA of a generated ray; false when it does not start
-__device__ __forceinline__ bool hp_begin(const HierScene& H, const GridRegs& G, HierRay& r)
+__device__ __forceinline__ bool hp_begin(const HierScene& H, const GridRegs& G, LdsMailbox& mb, HierRay& r)
 {
     r.best = H.nt;
     r.inst = 0xFFFFFFFFu;
     r.in_inst = false;
     r.pit = r.pend = 0u;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) r.mb.e[j] = 0xFFFFFFFFu;
+    for (int j = 0; j < 8; ++j) mb[j][__lane_id()] = 0xFFFFFFFFu;
     bool flag = !(r.t < r.tterm);
     const f3 t1 = (G.bmin - r.org) * r.rcp;
     f3 tfar = (G.bmax - r.org) * r.rcp;
@@ -501,144 +518,174 @@ __device__ __forceinline__ bool hp_begin(const HierScene& H, const GridRegs& G, 
     const f3 entry = (tentry >= 0.f) ? r.org + rep(tentry + kEps) / r.rcp : r.org;
     f3 cf = (entry - G.bmin) * G.csr;
     cf = mk(floorf(cf.x), floorf(cf.y), floorf(cf.z));
-    r.tx = ((cf.x + (r.rcp.x > 0.f ? 1.f : 0.f)) * G.cs.x + G.bmin.x - r.org.x) * r.rcp.x;
-    r.ty = ((cf.y + (r.rcp.y > 0.f ? 1.f : 0.f)) * G.cs.y + G.bmin.y - r.org.y) * r.rcp.y;
-    r.tz = ((cf.z + (r.rcp.z > 0.f ? 1.f : 0.f)) * G.cs.z + G.bmin.z - r.org.z) * r.rcp.z;
-    r.cx = to_int_sat(cf.x);
-    r.cy = to_int_sat(cf.y);
-    r.cz = to_int_sat(cf.z);
-    flag = flag && (r.rcp.x > 0.f ? r.cx < G.rx : r.cx > -1) && (r.rcp.y > 0.f ? r.cy < G.ry : r.cy > -1) &&
-           (r.rcp.z > 0.f ? r.cz < G.rz : r.cz > -1);
+    const bool px = r.rcp.x > 0.f, py = r.rcp.y > 0.f, pz = r.rcp.z > 0.f;
+    r.tx = ((cf.x + (px ? 1.f : 0.f)) * G.cs.x + G.bmin.x - r.org.x) * r.rcp.x;
+    r.ty = ((cf.y + (py ? 1.f : 0.f)) * G.cs.y + G.bmin.y - r.org.y) * r.rcp.y;
+    r.tz = ((cf.z + (pz ? 1.f : 0.f)) * G.cs.z + G.bmin.z - r.org.z) * r.rcp.z;
+    const int cx = to_int_sat(cf.x), cy = to_int_sat(cf.y), cz = to_int_sat(cf.z);
+    flag = flag && (px ? cx < G.rx : cx > -1) && (py ? cy < G.ry : cy > -1) && (pz ? cz < G.rz : cz > -1);
     if (!flag) return false;
+    r.cell = (uint32_t)cx + (uint32_t)cy * (uint32_t)G.rx + (uint32_t)cz * ((uint32_t)G.rx * (uint32_t)G.ry);
+    r.cx = steps_left(px, G.rx, cx);
+    r.cy = steps_left(py, G.ry, cy);
+    r.cz = steps_left(pz, G.rz, cz);
     hp_top_cell(H, G, r);
     return true;
 }
 
-// one unit of work other than a triangle test (an object-grid step, an
-// instance set-up or a top-grid step); true when the ray is finished.
-// entered: an instance's object grid was entered (r.ot / r.dt set)
-__device__ __forceinline__ bool hp_unit(const HierScene& H, const GridRegs& G, HierRay& r, bool& entered)
+// the object DDA's step after a cell; true when the ray is finished
+__device__ __forceinline__ bool hp_obj_step(const HierScene& H, HierRay& r)
 {
-    if (r.in_inst) {
-        // the object DDA's step after a cell
-        const int d = min_dim(r.otx, r.oty, r.otz);
-        bool flag;
-        if (d == 0) {
-            flag = r.rayT > r.otx;
-            r.ocx += r.rt.x > 0.f ? 1 : -1;
-            r.otx += r.ocs.x * fabsf(r.rt.x);
-            flag = flag && (r.rt.x > 0.f ? r.ocx < r.rx : r.ocx > -1);
-        } else if (d == 1) {
-            flag = r.rayT > r.oty;
-            r.ocy += r.rt.y > 0.f ? 1 : -1;
-            r.oty += r.ocs.y * fabsf(r.rt.y);
-            flag = flag && (r.rt.y > 0.f ? r.ocy < r.ry : r.ocy > -1);
-        } else {
-            flag = r.rayT > r.otz;
-            r.ocz += r.rt.z > 0.f ? 1 : -1;
-            r.otz += r.ocs.z * fabsf(r.rt.z);
-            flag = flag && (r.rt.z > 0.f ? r.ocz < r.rz : r.ocz > -1);
-        }
-        if (flag) {
-            hp_obj_cell(H, r);
-            return false;
-        }
-        r.in_inst = false;
-        if (r.hit != H.nt && r.rayT < r.t && r.rayT >= r.te1 && r.rayT < r.tx1) {
-            r.t = r.rayT;
-            r.best = r.hit;
-            r.inst = r.ii;
-            // the distance only shrinks from here: an occlusion test against
-            // tstop is decided
-            if (r.t < r.tstop) return true;
-        }
+    const Axis a = min_axis(r.otx, r.oty, r.otz);
+    const float tc = pick(a, r.otx, r.oty, r.otz);
+    const uint32_t left = pick(a, r.ocx, r.ocy, r.ocz) - 1u;
+    if (r.rayT > tc && left != 0u) {
+        put(a, tc + pick(a, r.od.x, r.od.y, r.od.z), r.otx, r.oty, r.otz);
+        put(a, left, r.ocx, r.ocy, r.ocz);
+        r.ocell += (uint32_t)pick(a, r.sx, r.sy, r.sz);
+        hp_obj_cell(H, r);
         return false;
     }
-    // the next instance of the top cell that the ray meets
-    while (r.it < r.end) {
-        const uint32_t ii = H.inst_refs[r.it];
-        ++r.it;
-        if (mailbox_seen(r.mb, ii)) continue;
-        const InstanceDev I = H.inst[ii];
-        const InstGrid Q = H.inst_grid[ii];
-        const f3 b1 = (mk(I.bmin[0], I.bmin[1], I.bmin[2]) - r.org) * r.rcp;
-        f3 bm = (mk(I.bmax[0], I.bmax[1], I.bmax[2]) - r.org) * r.rcp;
-        const f3 bn = vmin(b1, bm);
-        bm = vmax(b1, bm);
-        const float te1 = fmaxf(fmaxf(bn.x, bn.y), bn.z);
-        const float tx1 = fminf(fminf(bm.x, bm.y), bm.z);
-        if (!(tx1 > te1 && tx1 >= 0.f && te1 < r.t)) continue;
-        f3 ot, rt;
-        instance_ray(I, r.org, r.rcp, ot, rt);
-        const GridRegs O = inst_grid_regs(Q);
-        const f3 g1 = (O.bmin - ot) * rt;
-        f3 gf = (O.bmax - ot) * rt;
-        const f3 gn = vmin(g1, gf);
-        gf = vmax(g1, gf);
-        const float tentry = fmaxf(fmaxf(gn.x, gn.y), gn.z);
-        const float texit = fminf(fminf(gf.x, gf.y), gf.z);
-        bool flag = texit > tentry && texit >= 0.f && tentry < r.t;
-        const f3 entry = (tentry >= 0.f) ? ot + rep(tentry + kEps) / rt : ot;
-        f3 cf = (entry - O.bmin) * O.csr;
-        cf = mk(floorf(cf.x), floorf(cf.y), floorf(cf.z));
-        cf.x = rt.x > 0.f ? fminf((float)O.rx - 1.f, cf.x) : fmaxf(cf.x, 0.f);
-        cf.y = rt.y > 0.f ? fminf((float)O.ry - 1.f, cf.y) : fmaxf(cf.y, 0.f);
-        cf.z = rt.z > 0.f ? fminf((float)O.rz - 1.f, cf.z) : fmaxf(cf.z, 0.f);
-        const int ocx = to_int_sat(cf.x), ocy = to_int_sat(cf.y), ocz = to_int_sat(cf.z);
-        flag = flag && (rt.x > 0.f ? ocx < O.rx : ocx > -1) && (rt.y > 0.f ? ocy < O.ry : ocy > -1) &&
-               (rt.z > 0.f ? ocz < O.rz : ocz > -1);
-        if (!flag) continue;          // no object cell is stepped: no hit from this instance
+    r.in_inst = false;
+    if (r.rayT < r.t && r.rayT >= r.te1 && r.rayT < r.tx1) {     // rayT starts at t: below it there is a hit
+        r.t = r.rayT;
+        r.best = r.hit;
+        r.inst = r.ii;
+        // the distance only shrinks from here: an occlusion test against
+        // tstop is decided
+        return r.t < r.tstop;
+    }
+    return false;
+}
+
+// the ray outside the objects: the next instance of the top cell that it meets,
+// or the step to the next top cell; true when the ray is finished.  entered: an
+// instance's object grid was entered (r.ot / r.dt set).  The instances that
+// the ray has visited or whose boxes it misses are passed in a loop of their
+// own, so that the lanes that meet one move into object space together.
+// Of the move's 18 divisions, those by the ray's reciprocal direction and
+// by the object-space one go through their correctly rounded reciprocals where
+// the operands are in range (InstanceDev.short_div: the rotation's entries).
+__device__ __forceinline__ bool hp_enter(const HierScene& H, const GridRegs& G, LdsMailbox& mb, HierRay& r,
+                                         bool& entered)
+{
+    uint32_t ii = 0xFFFFFFFFu;
+#pragma unroll 1
+    for (uint32_t m = 0; m < kTopSteps; ++m) {
+        while (r.it < r.end) {
+            const uint32_t id = H.inst_refs[r.it];
+            ++r.it;
+            uint32_t& seen = mb[id & 7u][__lane_id()];
+            if (seen == id) continue;
+            seen = id;
+            const InstanceDev& I = H.inst[id];
+            const f3 b1 = (mk(I.bmin[0], I.bmin[1], I.bmin[2]) - r.org) * r.rcp;
+            f3 bm = (mk(I.bmax[0], I.bmax[1], I.bmax[2]) - r.org) * r.rcp;
+            const f3 bn = vmin(b1, bm);
+            bm = vmax(b1, bm);
+            const float te1 = fmaxf(fmaxf(bn.x, bn.y), bn.z);
+            const float tx1 = fminf(fminf(bm.x, bm.y), bm.z);
+            if (tx1 > te1 && tx1 >= 0.f && te1 < r.t) {
+                ii = id;
+                r.te1 = te1;
+                r.tx1 = tx1;
+                break;
+            }
+        }
+        if (ii != 0xFFFFFFFFu) break;
+        // the top cell is done: the shadow stop, then the top DDA's step
+        if (r.t < r.tterm) return true;
+        const Axis a = min_axis(r.tx, r.ty, r.tz);
+        const float tc = pick(a, r.tx, r.ty, r.tz);
+        const uint32_t left = pick(a, r.cx, r.cy, r.cz) - 1u;
+        if (!(r.t > tc) || left == 0u) return true;
+        const float rc = pick(a, r.rcp.x, r.rcp.y, r.rcp.z);
+        const int st = pick(a, 1, G.rx, (int)((uint32_t)G.rx * (uint32_t)G.ry));
+        put(a, tc + pick(a, G.cs.x, G.cs.y, G.cs.z) * fabsf(rc), r.tx, r.ty, r.tz);
+        put(a, left, r.cx, r.cy, r.cz);
+        r.cell += rc > 0.f ? (uint32_t)st : 0u - (uint32_t)st;
+        hp_top_cell(H, G, r);
+    }
+    if (ii == 0xFFFFFFFFu) return false;
+    const InstanceDev I = H.inst[ii];
+    const InstGrid Q = H.inst_grid[ii];
+    const GridRegs O = inst_grid_regs(Q);
+    const f3 r0 = mk(I.irot0[0], I.irot0[1], I.irot0[2]);
+    const f3 r1 = mk(I.irot1[0], I.irot1[1], I.irot1[2]);
+    const f3 r2 = mk(I.irot2[0], I.irot2[1], I.irot2[2]);
+    const f3 ot = r0 * r.org.x + r1 * r.org.y + r2 * r.org.z + mk(I.it[0], I.it[1], I.it[2]);
+    f3 q0, q1, q2;
+    const f3 ar = vabs(r.rcp);
+    if (I.short_div && fminf(fminf(ar.x, ar.y), ar.z) >= kDivLow && fmaxf(fmaxf(ar.x, ar.y), ar.z) <= kDivHigh) {
+        const f3 y = mk(rcp_in_range(r.rcp.x), rcp_in_range(r.rcp.y), rcp_in_range(r.rcp.z));
+        q0 = mk(div_by_rcp(r0.x, r.rcp.x, y.x), div_by_rcp(r0.y, r.rcp.x, y.x), div_by_rcp(r0.z, r.rcp.x, y.x));
+        q1 = mk(div_by_rcp(r1.x, r.rcp.y, y.y), div_by_rcp(r1.y, r.rcp.y, y.y), div_by_rcp(r1.z, r.rcp.y, y.y));
+        q2 = mk(div_by_rcp(r2.x, r.rcp.z, y.z), div_by_rcp(r2.y, r.rcp.z, y.z), div_by_rcp(r2.z, r.rcp.z, y.z));
+    } else {
+        q0 = r0 / r.rcp.x;
+        q1 = r1 / r.rcp.y;
+        q2 = r2 / r.rcp.z;
+    }
+    const f3 d = q0 + q1 + q2;
+    const f3 rt = mk(rcp_rn(d.x), rcp_rn(d.y), rcp_rn(d.z));
+    const f3 dt = mk(rcp_rn(rt.x), rcp_rn(rt.y), rcp_rn(rt.z));
+    const f3 g1 = (O.bmin - ot) * rt;
+    f3 gf = (O.bmax - ot) * rt;
+    const f3 gn = vmin(g1, gf);
+    gf = vmax(g1, gf);
+    const float tentry = fmaxf(fmaxf(gn.x, gn.y), gn.z);
+    const float texit = fminf(fminf(gf.x, gf.y), gf.z);
+    bool flag = texit > tentry && texit >= 0.f && tentry < r.t;
+    f3 entry = ot;
+    if (tentry >= 0.f) {
+        const float te = tentry + kEps;
+        const f3 at = vabs(rt);
+        f3 q;
+        if (te <= kDivHigh && fminf(fminf(at.x, at.y), at.z) >= kDivLow &&
+            fmaxf(fmaxf(at.x, at.y), at.z) <= kDivHigh)
+            q = mk(div_by_rcp(te, rt.x, dt.x), div_by_rcp(te, rt.y, dt.y), div_by_rcp(te, rt.z, dt.z));
+        else
+            q = rep(te) / rt;
+        entry = ot + q;
+    }
+    f3 cf = (entry - O.bmin) * O.csr;
+    cf = mk(floorf(cf.x), floorf(cf.y), floorf(cf.z));
+    const bool px = rt.x > 0.f, py = rt.y > 0.f, pz = rt.z > 0.f;
+    cf.x = px ? fminf((float)O.rx - 1.f, cf.x) : fmaxf(cf.x, 0.f);
+    cf.y = py ? fminf((float)O.ry - 1.f, cf.y) : fmaxf(cf.y, 0.f);
+    cf.z = pz ? fminf((float)O.rz - 1.f, cf.z) : fmaxf(cf.z, 0.f);
+    const int ocx = to_int_sat(cf.x), ocy = to_int_sat(cf.y), ocz = to_int_sat(cf.z);
+    flag = flag && (px ? ocx < O.rx : ocx > -1) && (py ? ocy < O.ry : ocy > -1) && (pz ? ocz < O.rz : ocz > -1);
+    if (flag) {                   // else no object cell is stepped: no hit from this instance
         r.ii = ii;
-        r.te1 = te1;
-        r.tx1 = tx1;
         r.ot = ot;
-        r.rt = rt;
-        r.dt = mk(1.f / rt.x, 1.f / rt.y, 1.f / rt.z);
-        r.ocs = O.cs;
-        r.rx = O.rx;
-        r.ry = O.ry;
-        r.rz = O.rz;
-        r.base = Q.base;
-        r.otx = ((cf.x + (rt.x > 0.f ? 1.f : 0.f)) * O.cs.x + O.bmin.x - ot.x) * rt.x;
-        r.oty = ((cf.y + (rt.y > 0.f ? 1.f : 0.f)) * O.cs.y + O.bmin.y - ot.y) * rt.y;
-        r.otz = ((cf.z + (rt.z > 0.f ? 1.f : 0.f)) * O.cs.z + O.bmin.z - ot.z) * rt.z;
-        r.ocx = ocx;
-        r.ocy = ocy;
-        r.ocz = ocz;
+        r.dt = dt;
+        r.od = mk(O.cs.x * fabsf(rt.x), O.cs.y * fabsf(rt.y), O.cs.z * fabsf(rt.z));
+        r.rx = (uint32_t)O.rx;
+        r.ry = (uint32_t)O.ry;
+        r.rz = (uint32_t)O.rz;
+        const uint32_t rxy = r.rx * r.ry;
+        r.sx = px ? 1 : -1;
+        r.sy = py ? O.rx : -O.rx;
+        r.sz = pz ? (int)rxy : (int)(0u - rxy);
+        r.otx = ((cf.x + (px ? 1.f : 0.f)) * O.cs.x + O.bmin.x - ot.x) * rt.x;
+        r.oty = ((cf.y + (py ? 1.f : 0.f)) * O.cs.y + O.bmin.y - ot.y) * rt.y;
+        r.otz = ((cf.z + (pz ? 1.f : 0.f)) * O.cs.z + O.bmin.z - ot.z) * rt.z;
+        r.ocell = Q.base + (uint32_t)ocx + (uint32_t)ocy * r.rx + (uint32_t)ocz * rxy;
+        r.ocx = steps_left(px, O.rx, ocx);
+        r.ocy = steps_left(py, O.ry, ocy);
+        r.ocz = steps_left(pz, O.rz, ocz);
         r.rayT = r.t;
         r.hit = H.nt;
         r.in_inst = true;
         entered = true;
         hp_obj_cell(H, r);
-        return false;
     }
-    // the top cell is done: the shadow stop, then the top DDA's step
-    if (r.t < r.tterm) return true;
-    const int dm = min_dim(r.tx, r.ty, r.tz);
-    bool flag;
-    if (dm == 0) {
-        flag = r.t > r.tx;
-        r.cx += r.rcp.x > 0.f ? 1 : -1;
-        r.tx += G.cs.x * fabsf(r.rcp.x);
-        flag = flag && (r.rcp.x > 0.f ? r.cx < G.rx : r.cx > -1);
-    } else if (dm == 1) {
-        flag = r.t > r.ty;
-        r.cy += r.rcp.y > 0.f ? 1 : -1;
-        r.ty += G.cs.y * fabsf(r.rcp.y);
-        flag = flag && (r.rcp.y > 0.f ? r.cy < G.ry : r.cy > -1);
-    } else {
-        flag = r.t > r.tz;
-        r.cz += r.rcp.z > 0.f ? 1 : -1;
-        r.tz += G.cs.z * fabsf(r.rcp.z);
-        flag = flag && (r.rcp.z > 0.f ? r.cz < G.rz : r.cz > -1);
-    }
-    if (!flag) return true;
-    hp_top_cell(H, G, r);
     return false;
 }
 
 // one unit of work; true when the ray is finished
-__device__ __forceinline__ bool hp_step(const HierScene& H, const GridRegs& G, HierRay& r)
+__device__ __forceinline__ bool hp_step(const HierScene& H, const GridRegs& G, LdsMailbox& mb, HierRay& r)
 {
     if (r.pit < r.pend) {
         // one triangle of the object cell (MollerTrumboreIntersectionTest)
@@ -653,8 +700,9 @@ __device__ __forceinline__ bool hp_step(const HierScene& H, const GridRegs& G, H
         }
         return false;
     }
+    if (r.in_inst) return hp_obj_step(H, r);
     bool entered = false;
-    return hp_unit(H, G, r, entered);
+    return hp_enter(H, G, mb, r, entered);
 }
 
 // AmbientOcclusionRayGenerator of the hierarchy (TLGridHierarchyAOIntegrator.h:296-380)
@@ -670,7 +718,7 @@ struct GenAOHier {
     __device__ __forceinline__ uint32_t count() const { return npix * (uint32_t)ra.ao_samples; }
 
     // false: ray j has no traversal (its result is written); *traced: it counts as a ray
-    __device__ __forceinline__ bool gen(const HierScene& H, const GridRegs& G, uint32_t j, HierRay& r,
+    __device__ __forceinline__ bool gen(const HierScene& H, const GridRegs& G, LdsMailbox& mb, uint32_t j, HierRay& r,
                                         bool& traced) const
     {
         const uint32_t S_ = (uint32_t)ra.ao_samples;
@@ -697,7 +745,7 @@ struct GenAOHier {
         r.t = kFltMax;
         r.tterm = fmaxf(kShadowStop, ra.ao_dist);
         r.tstop = ra.ao_dist;
-        if (hp_begin(H, G, r)) return true;
+        if (hp_begin(H, G, mb, r)) return true;
         finish(H, j, r);
         return false;
     }
@@ -719,7 +767,7 @@ struct GenPrimaryHier {
 
     __device__ __forceinline__ uint32_t count() const { return npix; }
 
-    __device__ __forceinline__ bool gen(const HierScene& H, const GridRegs& G, uint32_t j, HierRay& r,
+    __device__ __forceinline__ bool gen(const HierScene& H, const GridRegs& G, LdsMailbox& mb, uint32_t j, HierRay& r,
                                         bool& traced) const
     {
         traced = true;
@@ -729,7 +777,7 @@ struct GenPrimaryHier {
         r.t = kFltMax;
         r.tterm = 0.f;
         r.tstop = -1.f;
-        if (hp_begin(H, G, r)) return true;
+        if (hp_begin(H, G, mb, r)) return true;
         finish(H, j, r);
         return false;
     }
@@ -757,6 +805,8 @@ template <class Gen>
 __global__ __launch_bounds__(kBlock) void k_hier_persist(HierScene H, Gen g, uint32_t* __restrict__ pool,
                                                          uint32_t refill, unsigned long long* ray_count)
 {
+    __shared__ LdsMailbox mailboxes[kBlock / kWave];
+    LdsMailbox& mb = mailboxes[__builtin_amdgcn_readfirstlane((int)threadIdx.x) / kWave];
     const GridRegs G = load_grid(H.top);
     const uint64_t lt = __lanemask_lt();
     const uint32_t nrays = g.count();
@@ -775,7 +825,7 @@ __global__ __launch_bounds__(kBlock) void k_hier_persist(HierScene H, Gen g, uin
                 j = base + (uint32_t)__popcll(idle & lt);
                 if (j < nrays) {
                     bool traced = false;
-                    live = g.gen(H, G, j, r, traced);
+                    live = g.gen(H, G, mb, j, r, traced);
                     started += traced ? 1u : 0u;
                 }
             }
@@ -784,7 +834,7 @@ __global__ __launch_bounds__(kBlock) void k_hier_persist(HierScene H, Gen g, uin
             if (exhausted) break;
             continue;
         }
-        if (live && hp_step(H, G, r)) {
+        if (live && hp_step(H, G, mb, r)) {
             live = false;
             g.finish(H, j, r);
         }
@@ -800,17 +850,25 @@ __global__ __launch_bounds__(kBlock) void k_hier_persist(HierScene H, Gen g, uin
 // k_hier_persist with the triangle tests batched across the wave (the
 // candidate references of each lane's current object cell, up to kBatchK per
 // lane and iteration, tested at full width against the lanes' object-space
-// rays kept in LDS; see wave_test_range).  A lane whose cell has no candidate
-// left takes one other unit per iteration.  Every ray's units and their order
-// are trace_hier's, so the outputs are the same.  Four waves per SIMD (at most
-// 128 VGPRs): render 25.6 -> 24.6 ms against the compiler's 144 VGPRs and three
-// waves, 31.6 ms with per-lane tests, on 10,000 instances at 1024^2 x 4 AO.
+// rays kept in LDS; see wave_test_range).  Every ray's units and their order
+// are trace_hier's, so the outputs are the same.
+//
+// VALU issue under divergence bounds it (14 % of the lanes active with every
+// unit in every iteration): the step into an object is some 300 instructions,
+// so lanes wait for it until kEnterMin of the wave do.  AO rays of 10,000
+// instances at 1024^2 x 4, frame with its camera rays: 21.6 ms before; short
+// divisions, steps by selects and the mailbox in LDS 14.7; two object steps an
+// iteration 13.6; entering at 8 / 16 / 24 / 32 / 40 lanes 13.7 / 13.3 / 12.9 /
+// 12.6 / 12.6; two top steps 12.3 (4: 12.4, 8: 12.5).  Five waves per SIMD
+// with 28 values spilled against four without: 12.6 and 12.9; six: 14.6.
 template <class Gen>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) void k_hier_persist_bt(HierScene H, Gen g, uint32_t* __restrict__ pool,
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5))) void k_hier_persist_bt(HierScene H, Gen g, uint32_t* __restrict__ pool,
                                                             uint32_t refill, unsigned long long* ray_count)
 {
     __shared__ WaveTests lds[kBlock / kWave];
+    __shared__ LdsMailbox mailboxes[kBlock / kWave];
     WaveTests& W = lds[__builtin_amdgcn_readfirstlane((int)threadIdx.x) / kWave];
+    LdsMailbox& mb = mailboxes[__builtin_amdgcn_readfirstlane((int)threadIdx.x) / kWave];
     const GridRegs G = load_grid(H.top);
     const uint32_t lane = __lane_id();
     const uint64_t lt = __lanemask_lt();
@@ -831,7 +889,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
                 j = base + (uint32_t)__popcll(idle & lt);
                 if (j < nrays) {
                     bool traced = false;
-                    live = g.gen(H, G, j, r, traced);
+                    live = g.gen(H, G, mb, j, r, traced);
                     started += traced ? 1u : 0u;
                 }
             }
@@ -841,12 +899,19 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
             continue;
         }
         bool done = false;
-        if (live && r.pit >= r.pend) {
-            bool entered = false;
-            done = hp_unit(H, G, r, entered);
-            if (entered) {
-                W.set_ray(lane, r.ot, r.dt, r.rayT);
+        if (live && r.in_inst && r.pit >= r.pend) {
+#pragma unroll 1
+            for (uint32_t m = 0; m < kObjSteps; ++m) {
+                done = hp_obj_step(H, r);
+                if (!r.in_inst || r.pit < r.pend) break;
             }
+        }
+        const bool out = live && !done && !r.in_inst;
+        const uint64_t outs = __ballot(out);
+        if (outs && ((uint32_t)__popcll(outs) >= kEnterMin || __ballot(live && r.in_inst) == 0ull) && out) {
+            bool entered = false;
+            done = hp_enter(H, G, mb, r, entered);
+            if (entered) W.set_ray(lane, r.ot, r.dt, r.rayT);
         }
         wave_test_range<false, kBatchK>(H.rec, H.prims, W, r.pit, r.pend, r.rayT, r.hit, lane, live && !done, wk);
         if (live && done) {

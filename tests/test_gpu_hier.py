@@ -2,6 +2,8 @@
 against the oracle (or_hier.c) on the same seeded scene: object grids, top
 grid, every cell list and reference bit-exact; closest hits (distance,
 triangle, instance), occlusion, and the hierarchy's AO frames exact."""
+import copy
+
 import numpy as np
 import pytest
 
@@ -141,6 +143,50 @@ def test_hier_ao_parity(inst_scene, pp, pers, refill):
         np.testing.assert_array_equal(e.primary_instances(), hio)
         np.testing.assert_array_equal(e.ao_occlusion(4), occo)
         np.testing.assert_array_equal(np.asarray(fb).reshape(-1, 3), fbo)
+    e.close()
+
+
+def _transformed(sc, ins, case):
+    """The scene with other instance transforms: rotation entries that are zero,
+    tiny (past the short divisions' range) or small with objects as small."""
+    sc, ins = copy.copy(sc), copy.copy(ins)
+    m = ins.matrices.copy()
+    if case == "zeros":
+        m[:, :3, :3] = np.eye(3, dtype=np.float32)
+        m[:, :3, 3] = -(ins.aabb_min + ins.aabb_max) / 2
+    elif case == "tiny":
+        m[::2, 0, 1] = 1e-25
+    else:
+        small = np.asarray(ins.objects) > 0          # object 0 is the room, which spans the top grid
+        m[small] = np.ldexp(m[small], case).astype(np.float32)
+        vid = np.unique(sc.idx[ins.obj_first[1]:])
+        sc.verts = sc.verts.copy()
+        sc.verts[:, vid] = np.ldexp(sc.verts[:, vid], case).astype(np.float32)
+    ins.matrices = m
+    return sc, ins
+
+
+@pytest.mark.parametrize("case", ["zeros", "tiny", -6, 3, -62])
+def test_hier_ao_transforms(inst_scene, case):
+    """The step into an object where its divisions take the short and the full
+    forms, in the batched and the per-lane persistent kernels."""
+    sc, ins = _transformed(*inst_scene, case)
+    e = _gpu(sc, ins)
+    h = _oracle(sc, ins)
+    c = sc.camera
+    e.set_camera(c["pos"], c["dir"], c["up"], c["fov"], 61, 47)
+    cam = O.camera(c["pos"], c["dir"], c["up"], c["fov"], 61, 47)
+    p = O.params(seed=SEED, ao_samples=3, ao_dist=1.7)
+    _, occo, hitso, hpo, hio = O.render_ao_hier(h, cam, p, sc.materials, sc.mat_idx, 0, None)
+    for pp, batch in ((0, 1), (0, 0), (1, 1), (1, 0)):
+        e.set_tuning(pp, 1, test_batch=batch)
+        e.render_frame(0, MODE_AO, jitter=1, ao_samples=3, ao_dist=1.7)
+        planes, prims = e.primary_hits()
+        np.testing.assert_array_equal(planes, hitso)
+        np.testing.assert_array_equal(prims, hpo)
+        np.testing.assert_array_equal(e.primary_instances(), hio)
+        np.testing.assert_array_equal(e.ao_occlusion(3), occo)
+    assert 0 < occo.mean() < 1
     e.close()
 
 
