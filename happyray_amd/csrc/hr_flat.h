@@ -340,6 +340,31 @@ __device__ __forceinline__ void set_ray(RayState& r, f3 org, f3 d)
 // 102,400 triangles stay at 1.5 ms: the L2's lines bound them, not the VALU.
 constexpr int kBatchK = 12;   // candidates a lane hands to its wave per iteration
 
+// Rays per wave of a launch of n rays that should spread over `blocks`
+// workgroups of four waves: 64, or fewer where 64 would leave some of them
+// empty.  The wave's other lanes take part in the tests only.  The time of a
+// small launch is the latency of its longest rays, and an iteration is shorter
+// with fewer rays in a wave (fewer kinds of steps and rounds of tests).
+inline uint32_t wave_lanes(size_t n, uint32_t blocks)
+{
+    const size_t waves = 4 * (size_t)blocks, per = (n + waves - 1) / waves;
+    return per < 1 ? 1u : (per > (size_t)kWave ? (uint32_t)kWave : (uint32_t)per);
+}
+
+inline uint32_t wave_blocks(size_t n, uint32_t lanes) { return (uint32_t)((n + 4 * (size_t)lanes - 1) / (4 * (size_t)lanes)); }
+
+inline uint32_t device_cus()
+{
+    static uint32_t cached = 0;
+    if (!cached) {
+        int dev = 0, cus = 0;
+        (void)hipGetDevice(&dev);
+        (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
+        cached = cus > 0 ? (uint32_t)cus : 256u;
+    }
+    return cached;
+}
+
 struct WaveTests {
     float4 o[kWave];          // a lane's ray: origin and current distance
     float4 d[kWave];          // direction, and (as bits) candidate - item of its run

@@ -23,18 +23,6 @@ using namespace trav;
 
 inline uint32_t cdiv_u(size_t a, size_t b) { return (uint32_t)((a + b - 1) / b); }
 
-uint32_t device_cus()
-{
-    static int cached = 0;
-    if (!cached) {
-        int dev = 0, cus = 0;
-        (void)hipGetDevice(&dev);
-        (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-        cached = cus > 0 ? cus : 256;
-    }
-    return (uint32_t)cached;
-}
-
 // ---------------------------------------------------------------------------
 // traversal
 // ---------------------------------------------------------------------------

@@ -90,14 +90,15 @@ __device__ __forceinline__ int roulette(const Mat& m, float rnum, f3& att, bool 
 template <bool kTwo>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) void k_trace_path(
     TraceScene S, RenderArgs ra, uint32_t npix, const float* __restrict__ hits,
-    const uint32_t* __restrict__ hit_prims, Shading sh, PathBuffers pb, uint32_t steps_max,
+    const uint32_t* __restrict__ hit_prims, Shading sh, PathBuffers pb, uint32_t lanes, uint32_t steps_max,
     unsigned long long* ray_count)
 {
     if (frame_skipped(ra)) return;
     __shared__ WaveTests lds[kBlock / kWave];
-    WaveTests& W = lds[__builtin_amdgcn_readfirstlane((int)threadIdx.x) / kWave];
-    const uint32_t pix = blockIdx.x * blockDim.x + threadIdx.x;
-    const bool in = pix < npix;   // every lane stays for add_work
+    const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)threadIdx.x) / kWave;
+    WaveTests& W = lds[wave];
+    const uint32_t pix = (blockIdx.x * (kBlock / kWave) + wave) * lanes + __lane_id();
+    const bool in = __lane_id() < lanes && pix < npix;   // every lane stays for the traces and add_work
     const uint32_t image = (uint32_t)image_of(ra);
     f3 org = rep(0.f), dir = rep(0.f);
     float t = kFltMax;
@@ -272,14 +273,15 @@ __device__ __forceinline__ bool on_light(f3 pos, f3 nrm, f3 e1, f3 e2, f3 p)
 // the rays of a wave through trace_wave (300 -> 112 us on the scene above)
 template <bool kTwo>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(6))) void k_path_shadow(
-    TraceScene S, RenderArgs ra, uint32_t npix, Shading sh, PathBuffers pb, uint32_t steps_max,
+    TraceScene S, RenderArgs ra, uint32_t npix, Shading sh, PathBuffers pb, uint32_t lanes, uint32_t steps_max,
     unsigned long long* ray_count)
 {
     if (frame_skipped(ra)) return;
     __shared__ WaveTests lds[kBlock / kWave];
-    WaveTests& W = lds[__builtin_amdgcn_readfirstlane((int)threadIdx.x) / kWave];
-    const uint32_t pix = blockIdx.x * blockDim.x + threadIdx.x;
-    const bool in = pix < npix;   // every lane stays for add_work
+    const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)threadIdx.x) / kWave;
+    WaveTests& W = lds[wave];
+    const uint32_t pix = (blockIdx.x * (kBlock / kWave) + wave) * lanes + __lane_id();
+    const bool in = __lane_id() < lanes && pix < npix;   // every lane stays for the traces and add_work
     const float t = in ? pb.end[6 * (size_t)npix + pix] : kFltMax;
     f3 ls = rep(0.f), dl = rep(0.f);
     bool traced = false;
@@ -426,14 +428,16 @@ void launch_path_multi(const TraceScene& S, const CameraDev& cam, const RenderAr
 {
     const uint32_t npix = (uint32_t)cam.res_x * (uint32_t)cam.res_y;
     const dim3 g(blocks_for(npix)), b(kBlock);
+    const uint32_t pl = wave_lanes(npix, 4 * device_cus()), sl = wave_lanes(npix, 2 * device_cus());
+    const dim3 gp(wave_blocks(npix, pl)), gs(wave_blocks(npix, sl));
     if (S.two_level) {
-        hipLaunchKernelGGL(k_trace_path<true>, g, b, 0, s, S, ra, npix, hits, hit_prims, sh, pb, steps_max,
+        hipLaunchKernelGGL(k_trace_path<true>, gp, b, 0, s, S, ra, npix, hits, hit_prims, sh, pb, pl, steps_max,
                            ray_count);
-        hipLaunchKernelGGL(k_path_shadow<true>, g, b, 0, s, S, ra, npix, sh, pb, steps_max, ray_count);
+        hipLaunchKernelGGL(k_path_shadow<true>, gs, b, 0, s, S, ra, npix, sh, pb, sl, steps_max, ray_count);
     } else {
-        hipLaunchKernelGGL(k_trace_path<false>, g, b, 0, s, S, ra, npix, hits, hit_prims, sh, pb, steps_max,
+        hipLaunchKernelGGL(k_trace_path<false>, gp, b, 0, s, S, ra, npix, hits, hit_prims, sh, pb, pl, steps_max,
                            ray_count);
-        hipLaunchKernelGGL(k_path_shadow<false>, g, b, 0, s, S, ra, npix, sh, pb, steps_max, ray_count);
+        hipLaunchKernelGGL(k_path_shadow<false>, gs, b, 0, s, S, ra, npix, sh, pb, sl, steps_max, ray_count);
     }
     if (after_trace) (void)hipEventRecord(after_trace, s);
     hipLaunchKernelGGL(k_path_direct, g, b, 0, s, S, ra, npix, sh, pb);

@@ -153,6 +153,60 @@ struct GenBatch {
 // the persistent kernel
 // ---------------------------------------------------------------------------
 
+// How a wave of the batched kernels gets its rays.  Its first `lanes` lanes hold
+// rays; where there are too few rays to fill every wave slot of the GPU the
+// host gives each wave fewer than 64, and the other lanes only take part in the
+// tests (a wave's iteration costs less with fewer rays, and more waves hide
+// each other's latency).  The first rays are the wave's own run of the launch,
+// later ones come from *pool (which starts past the runs); a null pool means
+// that the runs hold every ray.
+struct RayFetch {
+    uint64_t slots;
+    uint32_t first;
+    bool started;
+
+    __device__ __forceinline__ RayFetch(uint32_t lanes, uint32_t wave)
+        : slots(lanes < (uint32_t)kWave ? (1ull << lanes) - 1ull : ~0ull),
+          first((blockIdx.x * (kBlock / kWave) + wave) * lanes), started(false)
+    {
+    }
+
+    // the first of as many rays as there are idle slots
+    __device__ __forceinline__ uint32_t next(uint32_t* pool, uint64_t idle, uint32_t nrays, bool& exhausted)
+    {
+        const uint32_t n = (uint32_t)__popcll(idle);
+        uint32_t base = first;
+        if (started) {
+            base = 0;
+            if (__lane_id() == 0) base = atomicAdd(pool, n);
+            base = (uint32_t)__builtin_amdgcn_readfirstlane((int)base);
+        }
+        started = true;
+        exhausted = pool == nullptr || base >= nrays || n >= nrays - base;
+        return base;
+    }
+};
+
+// rays per wave and workgroups of a launch of n rays
+struct RayLaunch {
+    uint32_t lanes, blocks, refill;
+    bool pooled;
+};
+
+inline RayLaunch ray_launch(uint32_t n, uint32_t blocks_max, uint32_t refill)
+{
+    RayLaunch l;
+    // one wave per SIMD: 4096 occlusion rays take 59 us so, 92 and 161 us with two
+    // and six waves of fewer rays; 1,000 rays of one per wave 52 us (64: 78 us)
+    l.lanes = wave_lanes(n, device_cus());
+    const uint32_t need = wave_blocks(n, l.lanes);
+    l.pooled = need > blocks_max;
+    l.blocks = l.pooled ? blocks_max : need;
+    l.refill = refill * l.lanes / (uint32_t)kWave;
+    if (l.refill < 1u) l.refill = 1u;
+    return l;
+}
+
 // at most 64 VGPRs, so eight waves per SIMD hide the gathers' latency
 // (AO 3.19 -> 3.12 ms against the compiler's 70 VGPRs and seven waves).  The
 // leaf cell sizes of a top-cell visit are divided here, not read from the
@@ -226,12 +280,14 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8))) voi
 
 template <bool kTwo, bool kAny, class Gen, int kK>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(6))) void k_persist_bt(
-    TraceScene S, Gen gen, uint32_t nrays, uint32_t* __restrict__ pool, uint32_t refill, uint32_t steps_max,
-    unsigned long long* ray_count, unsigned long long* stats)
+    TraceScene S, Gen gen, uint32_t nrays, uint32_t* __restrict__ pool, uint32_t lanes, uint32_t refill,
+    uint32_t steps_max, unsigned long long* ray_count, unsigned long long* stats)
 {
     if (gen.skipped()) return;
     __shared__ WaveTests lds[kBlock / kWave];
-    WaveTests& W = lds[__builtin_amdgcn_readfirstlane((int)threadIdx.x) / kWave];
+    const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)threadIdx.x) / kWave;
+    WaveTests& W = lds[wave];
+    RayFetch fetch(lanes, wave);
     const GridRegs G = load_grid(S.gp);
     const uint32_t lane = __lane_id();
     const uint64_t lt = __lanemask_lt();
@@ -241,14 +297,10 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(6))) voi
     bool live = false;
     bool exhausted = false;
     while (true) {
-        const uint64_t idle = __ballot(!live);
-        const uint32_t nidle = (uint32_t)__popcll(idle);
-        if (!exhausted && (nidle >= refill || idle == ~0ull)) {
-            uint32_t base = 0;
-            if (lane == 0) base = atomicAdd(pool, nidle);
-            base = __shfl(base, 0, kWave);
-            if (base + nidle >= nrays) exhausted = true;
-            if (!live) {
+        const uint64_t idle = __ballot(!live) & fetch.slots;
+        if (!exhausted && ((uint32_t)__popcll(idle) >= refill || idle == fetch.slots)) {
+            const uint32_t base = fetch.next(pool, idle, nrays, exhausted);
+            if (!live && lane < lanes) {
                 j = base + (uint32_t)__popcll(idle & lt);
                 if (j < nrays) {
                     const bool ok = gen.start(j, r, S);
@@ -404,7 +456,7 @@ __global__ __launch_bounds__(kBlock) void k_persist_multi(const SceneDesc* __res
 template <bool kAny>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5))) void k_persist_multi_bt(
     const SceneDesc* __restrict__ scenes, const RayBatchDev* __restrict__ batches, const uint32_t* __restrict__ prefix,
-    uint32_t nb, uint32_t nrays, uint32_t* __restrict__ pool, uint32_t refill, uint32_t steps_max,
+    uint32_t nb, uint32_t nrays, uint32_t* __restrict__ pool, uint32_t lanes, uint32_t refill, uint32_t steps_max,
     unsigned long long* ray_count, unsigned long long* stats)
 {
     __shared__ WaveTests lds[kBlock / kWave];
@@ -412,6 +464,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5))) voi
     __shared__ const uint32_t* prims[kBlock];
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)threadIdx.x) / kWave;
     WaveTests& W = lds[wave];
+    RayFetch fetch(lanes, wave);
     const float4* const* own_rec = recs + wave * kWave;
     const uint32_t* const* own_prims = prims + wave * kWave;
     const uint32_t lane = __lane_id();
@@ -424,14 +477,10 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5))) voi
     bool live = false;
     bool exhausted = false;
     while (true) {
-        const uint64_t idle = __ballot(!live);
-        const uint32_t nidle = (uint32_t)__popcll(idle);
-        if (!exhausted && (nidle >= refill || idle == ~0ull)) {
-            uint32_t base = 0;
-            if (lane == 0) base = atomicAdd(pool, nidle);
-            base = __shfl(base, 0, kWave);
-            if (base + nidle >= nrays) exhausted = true;
-            if (!live) {
+        const uint64_t idle = __ballot(!live) & fetch.slots;
+        if (!exhausted && ((uint32_t)__popcll(idle) >= refill || idle == fetch.slots)) {
+            const uint32_t base = fetch.next(pool, idle, nrays, exhausted);
+            if (!live && lane < lanes) {
                 j = base + (uint32_t)__popcll(idle & lt);
                 if (j < nrays) {
                     uint32_t lo = 0, hi = nb;            // prefix[lo] <= j < prefix[hi]
@@ -737,16 +786,16 @@ void launch(const TraceScene& S, const Gen& gen, uint32_t nrays, uint32_t* pool,
             unsigned long long* ray_count, unsigned long long* stats, hipStream_t s, const PersistOpts& o)
 {
     if (nrays == 0) return;
-    fill_u32(pool, 0u, 1, nullptr, 1, s);
     const uint32_t need = (nrays + kBlock - 1) / kBlock;
     if (o.batch) {
         auto kern = k_persist_bt<kTwo, kAny, Gen, kBatchK>;
-        uint32_t blocks = persistent_blocks(kern);
-        if (blocks > need) blocks = need;
-        hipLaunchKernelGGL(kern, dim3(blocks), dim3(kBlock), 0, s, S, gen, nrays, pool, refill, o.steps, ray_count,
-                           stats);
+        const RayLaunch l = ray_launch(nrays, persistent_blocks(kern), refill);
+        if (l.pooled) fill_u32(pool, l.blocks * (kBlock / kWave) * l.lanes, 1, nullptr, 1, s);
+        hipLaunchKernelGGL(kern, dim3(l.blocks), dim3(kBlock), 0, s, S, gen, nrays, l.pooled ? pool : nullptr, l.lanes,
+                           l.refill, o.steps, ray_count, stats);
         return;
     }
+    fill_u32(pool, 0u, 1, nullptr, 1, s);
     auto kern = o.fuse ? k_persist<kTwo, kAny, Gen, true> : k_persist<kTwo, kAny, Gen, false>;
     uint32_t blocks = o.fuse ? persistent_blocks(k_persist<kTwo, kAny, Gen, true>)
                              : persistent_blocks(k_persist<kTwo, kAny, Gen, false>);
@@ -816,7 +865,6 @@ void persist_multi(const SceneDesc* scenes, const RayBatchDev* batches, const ui
                    unsigned long long* ray_count, unsigned long long* stats, hipStream_t s, const PersistOpts& o)
 {
     if (nrays == 0 || nb == 0) return;
-    fill_u32(pool, 0u, 1, nullptr, 1, s);
     int dev = 0, cus = 0;
     (void)hipGetDevice(&dev);
     (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
@@ -824,17 +872,16 @@ void persist_multi(const SceneDesc* scenes, const RayBatchDev* batches, const ui
     uint32_t blocks = (uint32_t)cus * (blocks_per_cu ? blocks_per_cu : 1u);
     const uint32_t need = (nrays + kBlock - 1) / kBlock;
     if (o.batch) {
+        auto kern = anyhit ? k_persist_multi_bt<true> : k_persist_multi_bt<false>;
         if (blocks_per_cu == 0)
             blocks = anyhit ? persistent_blocks(k_persist_multi_bt<true>) : persistent_blocks(k_persist_multi_bt<false>);
-        if (blocks > need) blocks = need;
-        if (anyhit)
-            hipLaunchKernelGGL(k_persist_multi_bt<true>, dim3(blocks), dim3(kBlock), 0, s, scenes, batches, prefix, nb,
-                               nrays, pool, refill, o.steps, ray_count, stats);
-        else
-            hipLaunchKernelGGL(k_persist_multi_bt<false>, dim3(blocks), dim3(kBlock), 0, s, scenes, batches, prefix,
-                               nb, nrays, pool, refill, o.steps, ray_count, stats);
+        const RayLaunch l = ray_launch(nrays, blocks, refill);
+        if (l.pooled) fill_u32(pool, l.blocks * (kBlock / kWave) * l.lanes, 1, nullptr, 1, s);
+        hipLaunchKernelGGL(kern, dim3(l.blocks), dim3(kBlock), 0, s, scenes, batches, prefix, nb, nrays,
+                           l.pooled ? pool : nullptr, l.lanes, l.refill, o.steps, ray_count, stats);
         return;
     }
+    fill_u32(pool, 0u, 1, nullptr, 1, s);
     if (blocks_per_cu == 0) {
         blocks = anyhit ? persistent_blocks(k_persist_multi<true>) : persistent_blocks(k_persist_multi<false>);
     }

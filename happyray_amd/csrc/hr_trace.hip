@@ -109,13 +109,15 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(6))) voi
 template <bool kTwo>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(6))) void k_primary_wave(
     TraceScene S, CameraDev cam, RenderArgs ra, uint32_t npix, float* __restrict__ hits,
-    uint32_t* __restrict__ hit_prims, uint32_t steps_max, unsigned long long* ray_count)
+    uint32_t* __restrict__ hit_prims, uint32_t lanes, uint32_t steps_max, unsigned long long* ray_count)
 {
     if (frame_skipped(ra)) return;
     __shared__ WaveTests lds[kBlock / kWave];
-    WaveTests& W = lds[__builtin_amdgcn_readfirstlane((int)threadIdx.x) / kWave];
-    const uint32_t pix = blockIdx.x * blockDim.x + threadIdx.x;   // row order: tiles measured slower here
-    const bool active = pix < npix;
+    const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)threadIdx.x) / kWave;
+    WaveTests& W = lds[wave];
+    // row order: tiles measured slower here
+    const uint32_t pix = (blockIdx.x * (kBlock / kWave) + wave) * lanes + __lane_id();
+    const bool active = __lane_id() < lanes && pix < npix;
     count_rays(ray_count, active);
     Work wk;
     const GridRegs G = load_grid(S.gp);
@@ -257,15 +259,16 @@ template <bool kTwo>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) void k_pt_wave(TraceScene S, RenderArgs ra, uint32_t npix,
                                                     const float* __restrict__ hits,
                                                     const uint32_t* __restrict__ hit_prims, Shading sh,
-                                                    float* __restrict__ fb, uint32_t steps_max,
+                                                    float* __restrict__ fb, uint32_t lanes, uint32_t steps_max,
                                                     unsigned long long* ray_count)
 {
     if (frame_skipped(ra)) return;
     __shared__ WaveTests lds[kBlock / kWave];
     __shared__ float light_terms[6][kBlock];   // a vertex's light terms wait here across its shadow ray
-    WaveTests& W = lds[__builtin_amdgcn_readfirstlane((int)threadIdx.x) / kWave];
-    const uint32_t pix = blockIdx.x * blockDim.x + threadIdx.x;
-    const bool in = pix < npix;
+    const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)threadIdx.x) / kWave;
+    WaveTests& W = lds[wave];
+    const uint32_t pix = (blockIdx.x * (kBlock / kWave) + wave) * lanes + __lane_id();
+    const bool in = __lane_id() < lanes && pix < npix;
     const GridRegs G = load_grid(S.gp);
     PathState P;
     P.radiance = rep(0.f);
@@ -567,18 +570,6 @@ __global__ __launch_bounds__(kBlock) void k_trace_batch(TraceScene S, const floa
 
 inline uint32_t blocks_for(size_t n) { return (uint32_t)((n + kBlock - 1) / kBlock); }
 
-uint32_t device_cus()
-{
-    static int cached = 0;
-    if (!cached) {
-        int dev = 0, cus = 0;
-        (void)hipGetDevice(&dev);
-        (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-        cached = cus > 0 ? cus : 256;
-    }
-    return (uint32_t)cached;
-}
-
 }  // namespace
 
 void launch_primary(const TraceScene& S, const CameraDev& cam, const RenderArgs& ra, float* hits,
@@ -587,12 +578,13 @@ void launch_primary(const TraceScene& S, const CameraDev& cam, const RenderArgs&
 {
     const uint32_t npix = (uint32_t)cam.res_x * (uint32_t)cam.res_y;
     if (wave_steps) {
+        const uint32_t lanes = wave_lanes(npix, 2 * device_cus());
         if (S.two_level)
-            hipLaunchKernelGGL(k_primary_wave<true>, dim3(blocks_for(npix)), dim3(kBlock), 0, s, S, cam, ra, npix,
-                               hits, hit_prims, wave_steps, ray_count);
+            hipLaunchKernelGGL(k_primary_wave<true>, dim3(wave_blocks(npix, lanes)), dim3(kBlock), 0, s, S, cam, ra, npix,
+                               hits, hit_prims, lanes, wave_steps, ray_count);
         else
-            hipLaunchKernelGGL(k_primary_wave<false>, dim3(blocks_for(npix)), dim3(kBlock), 0, s, S, cam, ra, npix,
-                               hits, hit_prims, wave_steps, ray_count);
+            hipLaunchKernelGGL(k_primary_wave<false>, dim3(wave_blocks(npix, lanes)), dim3(kBlock), 0, s, S, cam, ra, npix,
+                               hits, hit_prims, lanes, wave_steps, ray_count);
         return;
     }
     const uint32_t slots = tiled_slots((uint32_t)cam.res_x, (uint32_t)cam.res_y);
@@ -635,12 +627,15 @@ void launch_pt(const TraceScene& S, const RenderArgs& ra, uint32_t npix, const f
                unsigned long long* ray_count, hipStream_t s, uint32_t wave_steps)
 {
     if (wave_steps) {
+        // all the waves that fit: 16,000 paths of four vertices 518 us so, 581 and
+        // 648 us with half and a quarter of them, 886 us with 64 paths a wave
+        const uint32_t lanes = wave_lanes(npix, 4 * device_cus());
         if (S.two_level)
-            hipLaunchKernelGGL(k_pt_wave<true>, dim3(blocks_for(npix)), dim3(kBlock), 0, s, S, ra, npix, hits,
-                               hit_prims, sh, fb, wave_steps, ray_count);
+            hipLaunchKernelGGL(k_pt_wave<true>, dim3(wave_blocks(npix, lanes)), dim3(kBlock), 0, s, S, ra, npix, hits,
+                               hit_prims, sh, fb, lanes, wave_steps, ray_count);
         else
-            hipLaunchKernelGGL(k_pt_wave<false>, dim3(blocks_for(npix)), dim3(kBlock), 0, s, S, ra, npix, hits,
-                               hit_prims, sh, fb, wave_steps, ray_count);
+            hipLaunchKernelGGL(k_pt_wave<false>, dim3(wave_blocks(npix, lanes)), dim3(kBlock), 0, s, S, ra, npix, hits,
+                               hit_prims, sh, fb, lanes, wave_steps, ray_count);
         return;
     }
     if (S.two_level)

@@ -8,7 +8,7 @@ import pytest
 
 import pyoracle as O
 from gpu_util import SEED, gpu_engine, oracle_grid, random_rays
-from happyray_amd import GRID_TWO_LEVEL, GRID_UNIFORM_EXACT, MODE_AO, Server, rayfile, scenes
+from happyray_amd import GRID_TWO_LEVEL, GRID_UNIFORM_EXACT, MODE_AO, MODE_PATH, Server, rayfile, scenes
 from happyray_amd.server import REQ_CLOSEST, REQ_OCCLUDED, REQ_PATH
 
 pytestmark = pytest.mark.gpu
@@ -60,3 +60,41 @@ def test_server_record_payloads():
         else:
             np.testing.assert_array_equal(ox, oy)
     srv.close()
+
+
+@pytest.mark.parametrize("n", [1, 5, 1024, 1025, 2049, 20001, 65535, 65537, 400001])
+@pytest.mark.parametrize("kind", [GRID_TWO_LEVEL, GRID_UNIFORM_EXACT])
+def test_launch_sizes(kind, n):
+    """From one ray per wave over waves that are partly filled to launches whose
+    waves fetch more rays: the batched kernels, the per-lane persistent ones and
+    the one-ray-per-lane kernels agree on every ray and path."""
+    sc = scenes.icosphere_cluster(n_spheres=6, subdiv=3)
+    e = gpu_engine(sc, kind, 1.0, 2.2)
+    e.set_lights(sc.lights)
+    org, d = random_rays(sc, n, seed=n)
+    out = []
+    for batch, pers in ((1, 1), (0, 1), (0, 0)):
+        e.set_tuning(test_batch=batch, persistent_secondary=pers)
+        out.append([*e.trace(org, d), e.occluded(org, d, 1.5), e.path_trace(org, d, 3)])
+    for o in out[1:]:
+        for a, b in zip(o, out[0]):
+            np.testing.assert_array_equal(np.asarray(a), np.asarray(b))
+    assert n < 1000 or 0.02 < out[0][2].mean() < 0.98
+    e.close()
+
+
+@pytest.mark.parametrize("res", [(1, 1), (9, 7), (130, 63), (257, 256), (700, 600)])
+def test_camera_kernels_agree_on_small_and_large_images(res):
+    sc = scenes.icosphere_cluster(n_spheres=6, subdiv=3)
+    e = gpu_engine(sc, GRID_TWO_LEVEL, 0.25, 2.2)
+    e.set_lights(sc.lights)
+    e.set_camera_dict(dict(sc.camera, res=res))
+    out = []
+    for pp in (0, 1, 3):
+        e.set_tuning(persistent_primary=pp)
+        out.append([e.render_frame(0, MODE_PATH, jitter=1, pt_depth=3), *e.primary_hits(),
+                    e.render_frame(0, MODE_AO, jitter=1, ao_samples=3, ao_dist=1.5)])
+    for o in out[1:]:
+        for a, b in zip(o, out[0]):
+            np.testing.assert_array_equal(np.asarray(a), np.asarray(b))
+    e.close()
