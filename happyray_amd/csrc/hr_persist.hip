@@ -158,38 +158,61 @@ struct GenBatch {
 // host gives each wave fewer than 64, and the other lanes only take part in the
 // tests (a wave's iteration costs less with fewer rays, and more waves hide
 // each other's latency).  The first rays are the wave's own run of the launch,
-// later ones come from *pool (which starts past the runs); a null pool means
-// that the runs hold every ray.
+// later runs of `chunk` rays (0: of what is idle) come from *pool, which starts
+// past the first runs; a null pool means that those hold every ray.
 struct RayFetch {
     uint64_t slots;
-    uint32_t first;
-    bool started;
+    uint32_t cur, end;        // what is left of the wave's run (the same in every lane)
+    bool last;                // no run comes after it
 
-    __device__ __forceinline__ RayFetch(uint32_t lanes, uint32_t wave)
-        : slots(lanes < (uint32_t)kWave ? (1ull << lanes) - 1ull : ~0ull),
-          first((blockIdx.x * (kBlock / kWave) + wave) * lanes), started(false)
+    __device__ __forceinline__ RayFetch(uint32_t lanes, uint32_t chunk, uint32_t wave, uint32_t nrays,
+                                        const uint32_t* pool)
+        : slots(lanes < (uint32_t)kWave ? (1ull << lanes) - 1ull : ~0ull)
     {
+        const uint32_t first = chunk ? chunk : lanes;
+        take((blockIdx.x * (kBlock / kWave) + wave) * first, first, nrays);
+        last = last || pool == nullptr;
     }
 
-    // the first of as many rays as there are idle slots
-    __device__ __forceinline__ uint32_t next(uint32_t* pool, uint64_t idle, uint32_t nrays, bool& exhausted)
+    __device__ __forceinline__ void take(uint32_t base, uint32_t n, uint32_t nrays)
     {
-        const uint32_t n = (uint32_t)__popcll(idle);
-        uint32_t base = first;
-        if (started) {
-            base = 0;
-            if (__lane_id() == 0) base = atomicAdd(pool, n);
-            base = (uint32_t)__builtin_amdgcn_readfirstlane((int)base);
+        last = base >= nrays || n >= nrays - base;
+        cur = base < nrays ? base : nrays;
+        end = last ? nrays : base + n;
+    }
+
+    // the ray of the idle slot of the given rank, or nrays; the wave is exhausted
+    // when its run is empty and is the last
+    __device__ __forceinline__ uint32_t next(uint32_t* pool, uint32_t chunk, uint64_t idle, uint32_t rank,
+                                             uint32_t nrays, bool& exhausted)
+    {
+        const uint32_t want = (uint32_t)__popcll(idle);
+        const uint32_t n0 = want < end - cur ? want : end - cur;
+        uint32_t j = rank < n0 ? cur + rank : nrays;
+        cur += n0;
+        if (n0 < want && !last) {
+            uint32_t base = 0;
+            const uint32_t c = chunk ? chunk : want - n0;
+            if (__lane_id() == 0) base = atomicAdd(pool, c);
+            take((uint32_t)__builtin_amdgcn_readfirstlane((int)base), c, nrays);
+            const uint32_t n1 = want - n0 < end - cur ? want - n0 : end - cur;
+            if (rank >= n0 && rank - n0 < n1) j = cur + (rank - n0);
+            cur += n1;
         }
-        started = true;
-        exhausted = pool == nullptr || base >= nrays || n >= nrays - base;
-        return base;
+        exhausted = cur == end && last;
+        return j;
     }
 };
 
-// rays per wave and workgroups of a launch of n rays
+// Rays per wave and workgroups of a launch of n rays, and the rays of a run: an
+// eighth of a wave's share in whole waves, at most 256.  The counter's atomics
+// serialise at the memory side (12 ns each): 8.4M AO rays fetched 56 at a time
+// made 150,000 of them in 2 ms.  AO of 1M triangles 1.953 ms fetching what is
+// idle, 1.950 in runs of 64, 1.760 in runs of 128.  Where an eighth of the share
+// is less than a wave (1M rays: 20) what is idle is fetched (chunk 0): waves that
+// keep rays to start at the end of the launch cost more (0.93 -> 1.00 ms).
 struct RayLaunch {
-    uint32_t lanes, blocks, refill;
+    uint32_t lanes, blocks, refill, chunk;
     bool pooled;
 };
 
@@ -204,6 +227,11 @@ inline RayLaunch ray_launch(uint32_t n, uint32_t blocks_max, uint32_t refill)
     l.blocks = l.pooled ? blocks_max : need;
     l.refill = refill * l.lanes / (uint32_t)kWave;
     if (l.refill < 1u) l.refill = 1u;
+    l.chunk = 0;
+    if (l.pooled) {
+        const uint32_t c = n / (l.blocks * (kBlock / kWave) * 8u) / (uint32_t)kWave * (uint32_t)kWave;
+        l.chunk = c < 4u * (uint32_t)kWave ? c : 4u * (uint32_t)kWave;
+    }
     return l;
 }
 
@@ -280,14 +308,14 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8))) voi
 
 template <bool kTwo, bool kAny, class Gen, int kK>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(6))) void k_persist_bt(
-    TraceScene S, Gen gen, uint32_t nrays, uint32_t* __restrict__ pool, uint32_t lanes, uint32_t refill,
+    TraceScene S, Gen gen, uint32_t nrays, uint32_t* __restrict__ pool, uint32_t lanes, uint32_t chunk, uint32_t refill,
     uint32_t steps_max, unsigned long long* ray_count, unsigned long long* stats)
 {
     if (gen.skipped()) return;
     __shared__ WaveTests lds[kBlock / kWave];
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)threadIdx.x) / kWave;
     WaveTests& W = lds[wave];
-    RayFetch fetch(lanes, wave);
+    RayFetch fetch(lanes, chunk, wave, nrays, pool);
     const GridRegs G = load_grid(S.gp);
     const uint32_t lane = __lane_id();
     const uint64_t lt = __lanemask_lt();
@@ -299,9 +327,9 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(6))) voi
     while (true) {
         const uint64_t idle = __ballot(!live) & fetch.slots;
         if (!exhausted && ((uint32_t)__popcll(idle) >= refill || idle == fetch.slots)) {
-            const uint32_t base = fetch.next(pool, idle, nrays, exhausted);
+            const uint32_t got = fetch.next(pool, chunk, idle, (uint32_t)__popcll(idle & lt), nrays, exhausted);
             if (!live && lane < lanes) {
-                j = base + (uint32_t)__popcll(idle & lt);
+                j = got;
                 if (j < nrays) {
                     const bool ok = gen.start(j, r, S);
                     started += ok ? 1u : 0u;
@@ -471,7 +499,7 @@ __global__ __launch_bounds__(kBlock) void k_persist_multi(const SceneDesc* __res
 template <bool kAny>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5))) void k_persist_multi_bt(
     const SceneDesc* __restrict__ scenes, const RayBatchDev* __restrict__ batches, const uint32_t* __restrict__ prefix,
-    uint32_t nb, uint32_t nrays, uint32_t* __restrict__ pool, uint32_t lanes, uint32_t refill, uint32_t steps_max,
+    uint32_t nb, uint32_t nrays, uint32_t* __restrict__ pool, uint32_t lanes, uint32_t chunk, uint32_t refill, uint32_t steps_max,
     unsigned long long* ray_count, unsigned long long* stats)
 {
     __shared__ WaveTests lds[kBlock / kWave];
@@ -479,7 +507,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5))) voi
     __shared__ const uint32_t* prims[kBlock];
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)threadIdx.x) / kWave;
     WaveTests& W = lds[wave];
-    RayFetch fetch(lanes, wave);
+    RayFetch fetch(lanes, chunk, wave, nrays, pool);
     const float4* const* own_rec = recs + wave * kWave;
     const uint32_t* const* own_prims = prims + wave * kWave;
     const uint32_t lane = __lane_id();
@@ -494,9 +522,9 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5))) voi
     while (true) {
         const uint64_t idle = __ballot(!live) & fetch.slots;
         if (!exhausted && ((uint32_t)__popcll(idle) >= refill || idle == fetch.slots)) {
-            const uint32_t base = fetch.next(pool, idle, nrays, exhausted);
+            const uint32_t got = fetch.next(pool, chunk, idle, (uint32_t)__popcll(idle & lt), nrays, exhausted);
             if (!live && lane < lanes) {
-                j = base + (uint32_t)__popcll(idle & lt);
+                j = got;
                 if (j < nrays) {
                     uint32_t lo = 0, hi = nb;            // prefix[lo] <= j < prefix[hi]
                     while (hi - lo > 1) {
@@ -805,8 +833,8 @@ void launch(const TraceScene& S, const Gen& gen, uint32_t nrays, uint32_t* pool,
     if (o.batch) {
         auto kern = k_persist_bt<kTwo, kAny, Gen, kBatchK>;
         const RayLaunch l = ray_launch(nrays, persistent_blocks(kern), refill);
-        if (l.pooled) fill_u32(pool, l.blocks * (kBlock / kWave) * l.lanes, 1, nullptr, 1, s);
-        hipLaunchKernelGGL(kern, dim3(l.blocks), dim3(kBlock), 0, s, S, gen, nrays, l.pooled ? pool : nullptr, l.lanes,
+        if (l.pooled) fill_u32(pool, l.blocks * (kBlock / kWave) * (l.chunk ? l.chunk : l.lanes), 1, nullptr, 1, s);
+        hipLaunchKernelGGL(kern, dim3(l.blocks), dim3(kBlock), 0, s, S, gen, nrays, l.pooled ? pool : nullptr, l.lanes, l.chunk,
                            l.refill, o.steps, ray_count, stats);
         return;
     }
@@ -891,9 +919,9 @@ void persist_multi(const SceneDesc* scenes, const RayBatchDev* batches, const ui
         if (blocks_per_cu == 0)
             blocks = anyhit ? persistent_blocks(k_persist_multi_bt<true>) : persistent_blocks(k_persist_multi_bt<false>);
         const RayLaunch l = ray_launch(nrays, blocks, refill);
-        if (l.pooled) fill_u32(pool, l.blocks * (kBlock / kWave) * l.lanes, 1, nullptr, 1, s);
+        if (l.pooled) fill_u32(pool, l.blocks * (kBlock / kWave) * (l.chunk ? l.chunk : l.lanes), 1, nullptr, 1, s);
         hipLaunchKernelGGL(kern, dim3(l.blocks), dim3(kBlock), 0, s, scenes, batches, prefix, nb, nrays,
-                           l.pooled ? pool : nullptr, l.lanes, l.refill, o.steps, ray_count, stats);
+                           l.pooled ? pool : nullptr, l.lanes, l.chunk, l.refill, o.steps, ray_count, stats);
         return;
     }
     fill_u32(pool, 0u, 1, nullptr, 1, s);

@@ -62,7 +62,8 @@ def test_server_record_payloads():
     srv.close()
 
 
-@pytest.mark.parametrize("n", [1, 5, 1024, 1025, 2049, 20001, 65535, 65537, 400001])
+@pytest.mark.parametrize("n", [1, 5, 1024, 1025, 2049, 20001, 65535, 65537, 400001,
+                               3300001, 6800003])
 @pytest.mark.parametrize("kind", [GRID_TWO_LEVEL, GRID_UNIFORM_EXACT])
 def test_launch_sizes(kind, n):
     """From one ray per wave over waves that are partly filled to launches whose
