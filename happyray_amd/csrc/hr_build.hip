@@ -292,9 +292,9 @@ __device__ __forceinline__ uint32_t list_owner(uint32_t* mark, uint32_t lane, ui
 // in kPairSlices slices each, in place of one wave that the whole launch waits
 // for.  A slice has at least kSliceMin candidates, so that reading the 64
 // triangles again is a small part of its work.  Two ground triangles of a
-// 74-cells-wide exact grid (82,000 triangles): the whole frame with its two passes
-// 1718 -> 645 us, 640 us a pass before; 768 wall
-// triangles of a two-level grid of 20,480: write pass 12.6 -> 5.1 us.
+// 74-cells-wide exact grid (82,000 triangles): 640 us a pass before, rebuild and
+// frame 1718 -> 645 us; 768 wall triangles of a two-level grid of 20,480: write
+// pass 12.6 -> 5.1 us.
 constexpr uint32_t kPairsHeavy = 1024;     // candidates of a wave from which it is listed
 constexpr uint32_t kPairSlices = 32;
 constexpr uint32_t kSliceMin = 256;

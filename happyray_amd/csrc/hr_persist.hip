@@ -228,7 +228,7 @@ inline RayLaunch ray_launch(uint32_t n, uint32_t blocks_max, uint32_t refill)
     l.refill = refill * l.lanes / (uint32_t)kWave;
     if (l.refill < 1u) l.refill = 1u;
     l.chunk = 0;
-    if (l.pooled) {
+    if (l.pooled && n <= 0xFF000000u) {     // the counter runs past n by a run per wave: not past 32 bits
         const uint32_t c = n / (l.blocks * (kBlock / kWave) * 8u) / (uint32_t)kWave * (uint32_t)kWave;
         l.chunk = c < 4u * (uint32_t)kWave ? c : 4u * (uint32_t)kWave;
     }
