@@ -95,10 +95,12 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
 {
     if (frame_skipped(ra)) return;
     __shared__ WaveTests lds[kBlock / kWave];
+    __shared__ GroupTally tally;
+    tally.clear();
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)threadIdx.x) / kWave;
     WaveTests& W = lds[wave];
     const uint32_t pix = (blockIdx.x * (kBlock / kWave) + wave) * lanes + __lane_id();
-    const bool in = __lane_id() < lanes && pix < npix;   // every lane stays for the traces and add_work
+    const bool in = __lane_id() < lanes && pix < npix;   // every lane stays for the traces and the counts
     const uint32_t image = (uint32_t)image_of(ra);
     f3 org = rep(0.f), dir = rep(0.f);
     float t = kFltMax;
@@ -239,8 +241,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
             }
         }
     }
-    if (ray_count && traced) atomicAdd(ray_count, (unsigned long long)traced);
-    add_work(ra.stats, traced, wk);
+    tally.add(ray_count, ra.stats, traced, wk);
     if (!in) return;
     pb.end[pix] = e_hp.x;
     pb.end[(size_t)npix + pix] = e_hp.y;
@@ -278,10 +279,12 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(6))) voi
 {
     if (frame_skipped(ra)) return;
     __shared__ WaveTests lds[kBlock / kWave];
+    __shared__ GroupTally tally;
+    tally.clear();
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)threadIdx.x) / kWave;
     WaveTests& W = lds[wave];
     const uint32_t pix = (blockIdx.x * (kBlock / kWave) + wave) * lanes + __lane_id();
-    const bool in = __lane_id() < lanes && pix < npix;   // every lane stays for the traces and add_work
+    const bool in = __lane_id() < lanes && pix < npix;   // every lane stays for the traces and the counts
     const float t = in ? pb.end[6 * (size_t)npix + pix] : kFltMax;
     f3 ls = rep(0.f), dl = rep(0.f);
     bool traced = false;
@@ -321,8 +324,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(6))) voi
         if (st < 0.9999f) ls = rep(0.f);
         else dl = normalize(d2);
     }
-    count_rays(ray_count, traced);
-    add_work(ra.stats, traced ? 1u : 0u, wk);
+    tally.add(ray_count, ra.stats, traced ? 1u : 0u, wk);
     if (!in) return;
     st_rgb(pb.ls, pix, ls);
     st_rgb(pb.dir_ls, pix, dl);

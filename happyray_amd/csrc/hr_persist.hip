@@ -313,6 +313,8 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(6))) voi
 {
     if (gen.skipped()) return;
     __shared__ WaveTests lds[kBlock / kWave];
+    __shared__ GroupTally tally;
+    tally.clear();
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)threadIdx.x) / kWave;
     WaveTests& W = lds[wave];
     RayFetch fetch(lanes, chunk, wave, nrays, pool);
@@ -389,13 +391,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(6))) voi
             gen.finish(j, r, true, S);
         }
     }
-    if (ray_count) {
-        unsigned long long c = started;
-#pragma unroll
-        for (int d = kWave / 2; d >= 1; d >>= 1) c += __shfl_xor(c, d, kWave);
-        if (lane == 0 && c) atomicAdd(ray_count, c);
-    }
-    add_work(stats, started, wk);
+    tally.add(ray_count, stats, started, wk);
 }
 
 // The multi-scene kernel: the loop of k_persist with a per-lane scene.  A
@@ -505,6 +501,8 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5))) voi
     __shared__ WaveTests lds[kBlock / kWave];
     __shared__ const float4* recs[kBlock];
     __shared__ const uint32_t* prims[kBlock];
+    __shared__ GroupTally tally;
+    tally.clear();
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)threadIdx.x) / kWave;
     WaveTests& W = lds[wave];
     RayFetch fetch(lanes, chunk, wave, nrays, pool);
@@ -601,13 +599,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5))) voi
             }
         }
     }
-    if (ray_count) {
-        unsigned long long c = started;
-#pragma unroll
-        for (int d = kWave / 2; d >= 1; d >>= 1) c += __shfl_xor(c, d, kWave);
-        if (lane == 0 && c) atomicAdd(ray_count, c);
-    }
-    add_work(stats, started, wk);
+    tally.add(ray_count, stats, started, wk);
 }
 
 // ---------------------------------------------------------------------------

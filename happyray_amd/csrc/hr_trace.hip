@@ -113,12 +113,13 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(6))) voi
 {
     if (frame_skipped(ra)) return;
     __shared__ WaveTests lds[kBlock / kWave];
+    __shared__ GroupTally tally;
+    tally.clear();
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)threadIdx.x) / kWave;
     WaveTests& W = lds[wave];
     // row order: tiles measured slower here
     const uint32_t pix = (blockIdx.x * (kBlock / kWave) + wave) * lanes + __lane_id();
     const bool active = __lane_id() < lanes && pix < npix;
-    count_rays(ray_count, active);
     Work wk;
     const GridRegs G = load_grid(S.gp);
     f3 d0 = rep(0.f);
@@ -139,7 +140,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(6))) voi
         hits[6 * (size_t)npix + pix] = t;
         hit_prims[pix] = prim;
     }
-    add_work(ra.stats, active ? 1u : 0u, wk);
+    tally.add(ray_count, ra.stats, active ? 1u : 0u, wk);
 }
 
 // ---------------------------------------------------------------------------
@@ -264,6 +265,8 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
 {
     if (frame_skipped(ra)) return;
     __shared__ WaveTests lds[kBlock / kWave];
+    __shared__ GroupTally tally;
+    tally.clear();
     __shared__ float light_terms[6][kBlock];   // a vertex's light terms wait here across its shadow ray
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)threadIdx.x) / kWave;
     WaveTests& W = lds[wave];
@@ -337,8 +340,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
             }
         }
     }
-    if (ray_count && traced) atomicAdd(ray_count, (unsigned long long)traced);
-    add_work(ra.stats, traced, wk);
+    tally.add(ray_count, ra.stats, traced, wk);
     if (!in) return;
     fb_put(ra, fb + 3 * (size_t)pix, P.radiance.x, P.radiance.y, P.radiance.z);
 }

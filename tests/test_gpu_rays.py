@@ -3,12 +3,15 @@ SimpleRayTraverser.h:200-262, AORayExporter.h:50-68): record entry points
 equal the SoA ones, input rays through the simple integrator and the AO ray
 dump equal the oracle, and server requests carrying records equal the same
 requests carrying SoA planes."""
+import time
+
 import numpy as np
 import pytest
 
 import pyoracle as O
 from gpu_util import SEED, gpu_engine, oracle_grid, random_rays
-from happyray_amd import GRID_TWO_LEVEL, GRID_UNIFORM_EXACT, MODE_AO, MODE_PATH, Server, rayfile, scenes
+from happyray_amd import GRID_TWO_LEVEL, GRID_UNIFORM, GRID_UNIFORM_EXACT, MODE_AO, MODE_PATH, Server, rayfile, scenes
+from happyray_amd.devmem import DeviceArray
 from happyray_amd.server import REQ_CLOSEST, REQ_OCCLUDED, REQ_PATH
 
 pytestmark = pytest.mark.gpu
@@ -98,4 +101,67 @@ def test_camera_kernels_agree_on_small_and_large_images(res):
     for o in out[1:]:
         for a, b in zip(o, out[0]):
             np.testing.assert_array_equal(np.asarray(a), np.asarray(b))
+    e.close()
+
+
+@pytest.mark.parametrize("n", [1, 5, 255, 1000, 4097, 70001, 400001])
+@pytest.mark.parametrize("kind", [GRID_TWO_LEVEL, GRID_UNIFORM_EXACT])
+def test_counts_at_launch_sizes(kind, n):
+    """The batched kernels add a workgroup's ray and work counts together: the
+    totals are those of the kernels that add per wave, for closest hits,
+    occlusion rays, paths, and the frames of each integrator."""
+    sc = scenes.icosphere_cluster(n_spheres=6, subdiv=3)
+    e = gpu_engine(sc, kind, 1.0, 2.2)
+    e.set_lights(sc.lights)
+    w = max(1, int(n ** 0.5))
+    e.set_camera_dict(dict(sc.camera, res=(w, (n + w - 1) // w)))
+    org, d = random_rays(sc, n, seed=n)
+    got = []
+    for batch, pers, pp in ((1, 1, 3), (0, 1, 1), (0, 0, 0)):
+        e.set_tuning(test_batch=batch, persistent_secondary=pers, persistent_primary=pp)
+        counts = []
+        for step in (lambda: e.trace(org, d), lambda: e.occluded(org, d, 1.5),
+                     lambda: e.path_trace(org, d, 3),
+                     lambda: e.render_frame(0, MODE_PATH, jitter=1, pt_depth=3, collect_stats=True),
+                     lambda: e.render_frame(0, MODE_AO, jitter=1, ao_samples=1, ao_dist=1.5, collect_stats=True)):
+            e.work_stats()
+            r0 = e.timing().rays_traced
+            step()
+            ws = e.work_stats()
+            counts.append((e.timing().rays_traced - r0, ws.primary.rays, ws.primary.steps, ws.primary.tests,
+                           ws.secondary.rays, ws.secondary.steps, ws.secondary.tests))
+        got.append(counts)
+    assert got[0] == got[1] == got[2]
+    assert got[0][0][0] == n and got[0][1][0] == n
+    e.close()
+
+
+@pytest.mark.parametrize("n", [1000, 4000])
+def test_counters_do_not_bound_small_launches(n):
+    """1,000 rays are 1,000 waves of one ray each.  Adding the counts of every
+    wave to the device counters by itself takes 1.8 times as long as the per-lane
+    kernel of 16 waves takes for these short occlusion rays; by workgroup, 0.7."""
+    sc = scenes.random_soup(5, 7000, extent=10.0, size=0.3)
+    e = gpu_engine(sc, GRID_UNIFORM, 4.26, 2.0)
+    rng = np.random.default_rng(n)
+    d = rng.normal(0, 1, (3, n))
+    org = DeviceArray.from_host(rng.uniform(0, 10, (3, n)).astype(np.float32))
+    dirs = DeviceArray.from_host((d / np.linalg.norm(d, axis=0)).astype(np.float32))
+    occ = DeviceArray((n,), np.uint8)
+
+    def calls(k):
+        t = time.perf_counter()
+        for _ in range(k):
+            e.occluded_dev(org.value, dirs.value, n, 0.5, occ.value)
+        e.synchronize()
+        return (time.perf_counter() - t) / k
+
+    best = {}
+    for _ in range(8):                      # the two in turn, the least of each
+        for batch in (1, 0):
+            e.set_tuning(test_batch=batch)
+            calls(20)
+            best[batch] = min(best.get(batch, 1.0), calls(200))
+    print(f"{n} occlusion rays: batched {best[1] * 1e6:.1f} us, per lane {best[0] * 1e6:.1f} us", flush=True)
+    assert best[1] < 1.15 * best[0]
     e.close()
