@@ -32,6 +32,7 @@
 //    (vertex xyz), the record every later pass and the traversal read.
 #include "hr_build.h"
 #include "hr_hier.h"
+#include "hr_slices.h"
 
 namespace hr {
 
@@ -54,7 +55,7 @@ __global__ void k_reset(BuildStatus* st)
         st->overflow = 0u;
         st->n_pairs_eff = st->n_leaves_eff = st->n_leaf_pairs_eff = 0u;
         st->heavy = 0u;
-        st->pad = 0u;
+        st->refused = 0u;
     }
 }
 
@@ -282,22 +283,10 @@ __device__ __forceinline__ uint32_t list_owner(uint32_t* mark, uint32_t lane, ui
 {
     mark[lane] = 0u;
     wave_sync();
-    if (cnt && ex < j0 + kWave && ex + cnt > j0) mark[ex > j0 ? ex - j0 : 0u] = lane;
+    if (owns_in_step(ex, cnt, j0)) mark[ex > j0 ? ex - j0 : 0u] = lane;
     wave_sync();
     return wave_incl_max(mark[lane]);
 }
-
-// Waves of 64 triangles with many candidates (large triangles: walls, a ground)
-// are listed by the count pass and their candidates are spread over the launch
-// in kPairSlices slices each, in place of one wave that the whole launch waits
-// for.  A slice has at least kSliceMin candidates, so that reading the 64
-// triangles again is a small part of its work.  Two ground triangles of a
-// 74-cells-wide exact grid (82,000 triangles): 640 us a pass before, rebuild and
-// frame 1718 -> 645 us; 768 wall triangles of a two-level grid of 20,480: write
-// pass 12.6 -> 5.1 us.
-constexpr uint32_t kPairsHeavy = 1024;     // candidates of a wave from which it is listed
-constexpr uint32_t kPairSlices = 32;
-constexpr uint32_t kSliceMin = 256;
 
 // the list in device memory: BuildStatus.heavy entries {wave, candidates}, and
 // for exact insertion the pairs of every slice
@@ -305,12 +294,6 @@ struct PairList {
     uint2* waves;
     uint32_t* slice_pairs;
 };
-
-__device__ __forceinline__ uint32_t slice_len(uint32_t total)
-{
-    const uint32_t n = ((total + kPairSlices - 1u) / kPairSlices + kWave - 1u) / kWave * kWave;
-    return n < kSliceMin ? kSliceMin : n;
-}
 
 // scene of a global cell index: the last s with cell_base[s] <= c (cell
 // counts are positive, so the bases increase strictly)
@@ -360,14 +343,14 @@ __global__ __launch_bounds__(kBlock) void k_top_pairs(
     // this wave's items: itself, or every step-th slice of the list
     uint32_t item = own ? 0u : (blockIdx.x - own_blocks) * kWavesPerBlock + (uint32_t)wl;
     const uint32_t step = own ? 1u : (gridDim.x - own_blocks) * kWavesPerBlock;
-    const uint32_t items = own ? 1u : st->heavy * kPairSlices;
+    const uint32_t items = own ? 1u : kPass == kPairsSlices && st->refused ? 0u : st->heavy * kPairSlices;
     for (; item < items; item += step) {
         uint32_t wg = blockIdx.x * kWavesPerBlock + (uint32_t)wl, jb = 0, slice = 0;
         if (!own) {
             const uint2 e = list.waves[item / kPairSlices];
             wg = e.x;
             slice = item % kPairSlices;
-            jb = slice * slice_len(e.y);
+            jb = slice_begin(e.y, slice);
             if (jb >= e.y) {
                 if (kPass == kPairsSlices && lane == 0) list.slice_pairs[item] = 0u;
                 continue;
@@ -407,26 +390,27 @@ __global__ __launch_bounds__(kBlock) void k_top_pairs(
             tri_bounds(v0, v1, v2, lo, hi);
             if (kMulti && T.object_grids) object_box_cells(lo, hi, bmin, csr, rx, ry, rz, mn, mx);
             else box_cells(lo, hi, bmin, csr, rx, ry, rz, mn, mx);
-            cnt = (uint32_t)((mx[0] - mn[0]) * (mx[1] - mn[1]) * (mx[2] - mn[2]));
+            cnt = (uint32_t)(mx[0] - mn[0]) * (uint32_t)(mx[1] - mn[1]) * (uint32_t)(mx[2] - mn[2]);
         }
 
         if (!kExact && kPass == kPairsCount) {
             const uint32_t s = wave_sum(cnt);
             if (lane == 0) {
-                wave_counts[wg] = s;
+                wave_counts[wg] = pairs_count_or_refuse(s, s);
                 if (s >= kPairsHeavy) list.waves[atomicAdd(&st->heavy, 1u)] = make_uint2(wg, s);
             }
             return;
         }
 
         const uint32_t kcell_z = (uint32_t)rx * (uint32_t)ry;
-        const uint32_t inc = wave_incl_scan(cnt);
+        const uint32_t inc = wave_incl_scan_sat(cnt);
         const uint32_t ex = inc - cnt;
         const uint32_t total = (uint32_t)__builtin_amdgcn_readlane((int)inc, kWave - 1);
         if (own && total >= kPairsHeavy) {      // the list's slices do it
             if (kPass == kPairsCount && lane == 0) {
-                wave_counts[wg] = 0u;
-                list.waves[atomicAdd(&st->heavy, 1u)] = make_uint2(wg, total);
+                wave_counts[wg] = pairs_count_or_refuse(total, 0u);
+                if (total <= kPairsWaveMax) list.waves[atomicAdd(&st->heavy, 1u)] = make_uint2(wg, total);
+                else st->refused = 1u;
             }
             return;
         }
@@ -459,7 +443,7 @@ __global__ __launch_bounds__(kBlock) void k_top_pairs(
         uint32_t je = total, run = 0;
         if (kWrite) run = wave_offsets[wg];
         if (!own) {
-            je = total - jb < slice_len(total) ? total : jb + slice_len(total);
+            je = slice_end(total, slice);
             if (kWrite && kExact) {
                 // the pairs of the wave's slices before this one
                 const uint32_t c = lane < slice ? list.slice_pairs[item - slice + lane] : 0u;
@@ -477,8 +461,8 @@ __global__ __launch_bounds__(kBlock) void k_top_pairs(
             if (j < je) {
                 const uint32_t k = j - W.excl[o];
                 const uint32_t dxo = (uint32_t)W.dx[o], dyo = (uint32_t)W.dy[o];
-                const int ix = (int)(k % dxo), t = (int)(k / dxo);
-                const int iy = t % (int)dyo, iz = t / (int)dyo;
+                const uint32_t t = k / dxo;
+                const int ix = (int)(k % dxo), iy = (int)(t % dyo), iz = (int)(t / dyo);
                 const int x = W.lo[0][o] + ix, y = W.lo[1][o] + iy, z = W.lo[2][o] + iz;
                 id = W.id[o];
                 if (kMulti) key = W.cbase[o] + (uint32_t)x + (uint32_t)y * W.gx[o] + (uint32_t)z * W.gz[o];

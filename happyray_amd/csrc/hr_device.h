@@ -36,7 +36,7 @@ struct BuildStatus {
     uint32_t n_leaves_eff;
     uint32_t n_leaf_pairs_eff;
     uint32_t heavy;             // waves of triangles with many candidates, listed for the pair passes
-    uint32_t pad;
+    uint32_t refused;           // 1: a wave of triangles has more candidates than its list can have
 };
 
 // The per-frame selection of a captured frame (HIP graph): key frames, the

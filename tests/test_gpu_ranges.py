@@ -7,8 +7,8 @@ import numpy as np
 import pytest
 
 import pyoracle as O
-from gpu_util import gpu_engine, oracle_grid, random_rays
-from happyray_amd import GRID_TWO_LEVEL, GRID_UNIFORM, GRID_UNIFORM_EXACT, HappyRayError, scenes
+from gpu_util import SEED, assert_grid_equal, gpu_engine, oracle_grid, random_rays
+from happyray_amd import Engine, GRID_TWO_LEVEL, GRID_UNIFORM, GRID_UNIFORM_EXACT, HappyRayError, scenes
 from happyray_amd._lib import STATUS_NAMES
 
 pytestmark = pytest.mark.gpu
@@ -55,3 +55,33 @@ def test_leaf_counts_past_32_bits_are_refused():
     assert STATUS_NAMES[ex.value.status] == "HR_ERR_CAPACITY"
     sc.verts = keep
     gpu_engine(sc, GRID_TWO_LEVEL, 0.25, 2.2).close()
+
+
+def test_candidates_of_a_wave_past_32_bits_are_refused():
+    """64 walls across a grid of 8e7 cells have 5e9 candidate cells, past 2^32,
+    though the few cells that they cross would fit: an exact grid whose sum of
+    candidates wrapped would miss references.  The build refuses it, and the
+    engine builds and answers as before afterwards."""
+    rng = np.random.default_rng(3)
+    sc = scenes.random_soup(5, 80, extent=8.0, size=0.6)
+    v = sc.verts.reshape(3, -1, 3)
+    keep = sc.verts.copy()
+    corner = rng.integers(0, 2, (80, 3)) * 8.0
+    v[:, :, 0], v[:, :, 1] = corner.T, 8.0 - corner.T       # every triangle's box is the scene's
+    v[:, :, 2] = np.clip(v[:, :, 2], 0.0, 8.0)
+    sc.verts = np.ascontiguousarray(v.reshape(3, -1)).astype(np.float32)
+    e = Engine(seed=SEED)
+    for _ in range(2):
+        e.upload_scene(sc)
+        e.set_grid(GRID_UNIFORM_EXACT, 9.9e5, 1.0)
+        with pytest.raises(HappyRayError) as ex:
+            e.build_acc_struct()
+        assert STATUS_NAMES[ex.value.status] == "HR_ERR_CAPACITY"
+        e.upload(keep, None, 1.0, sc.idx)
+        e.set_grid(GRID_UNIFORM_EXACT, 5.0, 1.0)
+        e.build_acc_struct()
+        sc.verts, walls = keep, sc.verts
+        og = oracle_grid(sc, GRID_UNIFORM_EXACT, 5.0, 1.0)
+        assert_grid_equal(e, og)
+        sc.verts = walls
+    e.close()
