@@ -842,13 +842,6 @@ constexpr int kPrimaryKernels[3] = { 0, 1, 3 };
 // two rounds of trials: a kernel's first launch in a process, and the first
 // frame after a change, can take more than twice its steady time
 constexpr int kPrimaryTrials = 6;
-// kernel 0 is kept unless another takes less than its time by more than a
-// tenth: it runs on four workgroups per CU and leaves wave slots to the
-// neighbouring frame, which the trials, one frame at a time, do not see.  The
-// 1M-triangle soup's camera rays take 0.588 ms alone in kernel 0 and 0.589 in
-// kernel 3; four queued frames 11.0 ms with 0 and 11.3 with 3.  Where another
-// is chosen it is far ahead (heightfield 0.84 against 0.52 ms).
-constexpr float kPrimaryKeep = 1.1f;
 
 void resolve_primary_trial(hr_ctx* c)
 {
@@ -867,7 +860,6 @@ void resolve_primary_trial(hr_ctx* c)
         int b = 0;
         for (int k = 1; k < 3; ++k)
             if (c->pp_ms[k] < c->pp_ms[b]) b = k;
-        if (c->pp_ms[0] <= kPrimaryKeep * c->pp_ms[b]) b = 0;
         c->pp_choice = kPrimaryKernels[b];
     }
 }

@@ -325,7 +325,7 @@ typedef struct {
                                   six timed frames after the mesh, key frames, grid,
                                   camera or tuning change run 0, 1, 3, 0, 1, 3 (each waits
                                   for the one before it to finish), later frames the one
-                                  with the least time, or 0 if it is within a tenth of it
+                                  with the least time
                                   (hr_timing.primary_kernel shows which ran).  Same results
                                   either way; the instanced hierarchy takes 2 and 3 as 0 */
     int persistent_secondary;  /* AO rays and ray batches: 1 (default) persistent, 0 not */
