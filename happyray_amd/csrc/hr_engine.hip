@@ -994,7 +994,7 @@ hr_status enqueue_render(hr_ctx* c, hr_mode mode, int image_id, const hr_render_
                            c->stream);
         else
             hr::launch_pt(S, ra, npix, c->hits.p, c->hit_prims.p, sh, fb, rays, c->stream,
-                          pt_wave_steps(c));
+                          pt_wave_steps(c), hr::kPathsFrame);
         if (e_p2) HR_HIP(hipEventRecord(e_p2, c->stream));
     } else if (mode == HR_MODE_SIMPLE) {
         if (e_p2) HR_HIP(hipEventRecord(e_p2, c->stream));
@@ -1461,7 +1461,7 @@ hr_status path_trace_hits(hr_ctx* c, const float* hits, const uint32_t* prims, u
         hr::persist_pt(trace_scene(c), ra, n, hits, prims, sh, rgb, pool ? pool : c->pool.p,
                        (uint32_t)c->tuning.path_refill, (uint32_t)c->tuning.path_shade, c->ray_count.p, s);
     else
-        hr::launch_pt(trace_scene(c), ra, n, hits, prims, sh, rgb, c->ray_count.p, s, pt_wave_steps(c));
+        hr::launch_pt(trace_scene(c), ra, n, hits, prims, sh, rgb, c->ray_count.p, s, pt_wave_steps(c), hr::kPathsRays);
     HR_HIP(hipGetLastError());
     return HR_OK;
 }

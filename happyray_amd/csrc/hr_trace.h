@@ -89,10 +89,20 @@ void launch_ao_shade(const TraceScene& S, const RenderArgs& ra, uint32_t npix, c
                      hipStream_t s);
 // wave_steps > 0: the wave-cooperative kernel (batched candidate tests, up to
 // wave_steps grid steps per lane and batch); 0: one path per lane throughout.
-// The same image either way.
+// The same image either way.  Few paths are spread over blocks_per_cu workgroups
+// per CU (wave_lanes): kPathsFrame for the pixels of a frame, all the waves that
+// fit; kPathsRays, half of them, for paths from given rays, which several
+// contexts may trace at once.  Such paths share little, so a wave of few costs
+// nearly what a full one does and the GPU has no use for more waves than its
+// neighbours leave: 80,000 of four vertices on 20,480 triangles, three contexts in
+// turn, take 485 / 335 / 280 us a launch on all / half / a quarter of the waves
+// (alone 688 / 644 / 700; 16,000 alone 431 / 441 / 481).  A frame's are coherent:
+// 240x180 on two-level grids of 130,000 triangles 904 / 1010 / 1150 us alone, 440 /
+// 400 / 439 three in turn; 45,000 triangles 258 / 267 / 286 and 104 / 104 / 111.
+constexpr uint32_t kPathsFrame = 4, kPathsRays = 2;
 void launch_pt(const TraceScene& S, const RenderArgs& ra, uint32_t npix, const float* hits,
                const uint32_t* hit_prims, const Shading& sh, float* fb,
-               unsigned long long* ray_count, hipStream_t s, uint32_t wave_steps = 0);
+               unsigned long long* ray_count, hipStream_t s, uint32_t wave_steps, uint32_t blocks_per_cu);
 // current-frame normals: a * (1 - 0) + b * 0 per component, as the reference
 // uploads normals with coefficient 0 (src/RT/RTEngine.cu:209-210); a, b are
 // SoA key-frame blocks of nn normals

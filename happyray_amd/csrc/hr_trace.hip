@@ -626,12 +626,10 @@ void launch_ao_shade(const TraceScene& S, const RenderArgs& ra, uint32_t npix, c
 
 void launch_pt(const TraceScene& S, const RenderArgs& ra, uint32_t npix, const float* hits,
                const uint32_t* hit_prims, const Shading& sh, float* fb,
-               unsigned long long* ray_count, hipStream_t s, uint32_t wave_steps)
+               unsigned long long* ray_count, hipStream_t s, uint32_t wave_steps, uint32_t blocks_per_cu)
 {
     if (wave_steps) {
-        // all the waves that fit: 16,000 paths of four vertices 518 us so, 581 and
-        // 648 us with half and a quarter of them, 886 us with 64 paths a wave
-        const uint32_t lanes = wave_lanes(npix, 4 * device_cus());
+        const uint32_t lanes = wave_lanes(npix, blocks_per_cu * device_cus());
         if (S.two_level)
             hipLaunchKernelGGL(k_pt_wave<true>, dim3(wave_blocks(npix, lanes)), dim3(kBlock), 0, s, S, ra, npix, hits,
                                hit_prims, sh, fb, lanes, wave_steps, ray_count);
