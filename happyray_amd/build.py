@@ -82,5 +82,18 @@ def build(verbose=False):
     return LIB
 
 
+def build_checks():
+    """The GPU check of hr_math.h's short divisions (tests/math_check.hip), with the library's flags."""
+    tests = os.path.join(os.path.dirname(HERE), "tests")
+    lib = os.path.join(tests, "libmath_check.so")
+    cmd = [_hipcc(), "-shared", "-x", "hip", os.path.join(tests, "math_check.hip"), "-o", lib + ".tmp"] + FLAGS
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"building math_check failed:\n{r.stdout}\n{r.stderr}")
+    os.replace(lib + ".tmp", lib)
+    return lib
+
+
 if __name__ == "__main__":
     print(build(verbose=True))
+    print(build_checks())

@@ -59,7 +59,7 @@ HR_HD f3 normalize(f3 a) { return a * (1.f / sqrtf(dot(a, a))); }
 HR_HD float get(f3 a, int i) { return i == 0 ? a.x : (i == 1 ? a.y : a.z); }
 
 // 1 / x correctly rounded, as the division gives it, for 2^-125 <= |x| <= 2^125
-// (every such x was compared with the division): the hardware estimate and one
+// (a test compares every such x with the division): the hardware estimate and one
 // fused Newton step instead of the division's scaling and fix-up.
 __device__ __forceinline__ float rcp_in_range(float x)
 {
@@ -79,8 +79,12 @@ __device__ __forceinline__ float rcp_rn(float x)
 // a / b correctly rounded from y = 1 / b correctly rounded (Markstein, IBM J.
 // Res. Dev. 34(1), 1990: the residual of a quotient within one unit in the last
 // place, formed by a fused multiply-add, rounds it correctly; the first step
-// brings the quotient there).  For |b| in [2^-60, 2^60] and a either 0 or in
-// [2^-60, 2^60], where no step leaves the normal range.
+// brings the quotient there).  For |b| in [2^-60, 2^60] and |a| either 0 or in
+// [2^-60, 2^60], where no step leaves the normal range.  -0 over a positive b
+// gives +0: the callers add the quotient to a point or to two others of an
+// object-space direction, where only the direction's infinite reciprocal along an
+// axis that a singular transform collapses could see the sign, and both signs
+// step through the same cells there.
 __device__ __forceinline__ float div_by_rcp(float a, float b, float y)
 {
     float q = a * y;

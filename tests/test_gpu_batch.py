@@ -174,3 +174,43 @@ def test_autotune_choice_keeps_results():
     for e in engines:
         e.close()
     b.close()
+
+
+# With one workgroup per CU (256 CUs) rays beyond 65,536 of a kind come from the
+# counter: as lanes fall idle, in runs of 64 from 524,288 rays on, and in runs of
+# 256, the longest, from 2.1M on
+@pytest.mark.parametrize("total,refill", [(65537, 48), (120001, 1), (120001, 64), (700003, 48), (2300007, 48),
+                                          (2300007, 1)])
+def test_rays_from_the_counter(total, refill):
+    """Launches whose waves fetch rays past their first ones, over scenes with
+    ragged ray counts (runs that begin and end inside a scene's rays, scenes
+    within one run): every ray equals the one-ray-per-lane kernels of its scene
+    by itself."""
+    scs = scene_set()
+    rng = np.random.default_rng(total + refill)
+    cuts = np.sort(rng.choice(total - 1, len(scs) - 1, replace=False) + 1)
+    cuts[: 3] = (1, 3, 66)                                # scenes of a ray or two, and of one wave
+    counts = np.diff(np.concatenate([[0], np.sort(cuts), [total]]))
+    assert counts.min() >= 1 and counts.sum() == total
+    b = Batch()
+    b.set_scenes([(sc.verts, sc.idx) for sc in scs])
+    b.set_densities(0.25, 2.2)
+    b.build()
+    b.set_tuning(refill, 1)
+    items, engines = [], []
+    for s, (sc, n) in enumerate(zip(scs, counts)):
+        org, d = random_rays(sc, int(n), seed=total + s)
+        ext = float((sc.verts.max(1) - sc.verts.min(1)).max())
+        items += [(s, org, d, False, 0.0), (s, org, d, True, 0.3 * ext)]
+        e = single_engine(sc, 0.25, 2.2)
+        e.set_tuning(persistent_secondary=0)
+        engines.append(e)
+    rays = b.make_rays(items)
+    for _ in range(2):                                    # the counter starts anew
+        b.trace(rays)
+        b.synchronize()
+        check_rays(items, rays.results(), engines)
+    rays.free()
+    for e in engines:
+        e.close()
+    b.close()

@@ -225,3 +225,34 @@ def test_paths_of_several_contexts_share_the_gpu(mesh, kind, density):
     small, large = rate(80000), rate(240000)
     print(f"paths/us: {small * 1e-6:.0f} at 80,000 a launch, {large * 1e-6:.0f} at 240,000", flush=True)
     assert small > 0.63 * large
+
+
+# the flat kernel has at most six workgroups per CU, so rays past 393,216 come
+# from the counter: as lanes fall idle, in runs of 64 from 3.1M rays on, of 128
+# from 6.3M and of 256, the longest, from 12.6M
+@pytest.mark.parametrize("n,refills", [(450001, (1, 16, 48, 56, 64)), (3300001, (1, 64)), (6800003, (24,)),
+                                       (12900001, (56,))])
+@pytest.mark.parametrize("kind", [GRID_TWO_LEVEL, GRID_UNIFORM])
+def test_rays_from_the_counter(kind, n, refills):
+    """Launches whose waves fetch rays past their first ones, at several
+    thresholds: every ray and the work counts are the one-ray-per-lane kernels'."""
+    sc = scenes.icosphere_cluster(n_spheres=6, subdiv=3)
+    e = gpu_engine(sc, kind, 1.0, 2.2)
+    org, d = random_rays(sc, n, seed=n)
+
+    def query():
+        e.work_stats()
+        out = [*e.trace(org, d), e.occluded(org, d, 1.5)]
+        ws = e.work_stats().secondary
+        return out, (ws.rays, ws.steps, ws.tests)
+
+    e.set_tuning(persistent_secondary=0)
+    want, counts = query()
+    for refill in refills:
+        e.set_tuning(persistent_secondary=1, refill=refill)
+        got, c = query()
+        for a, b in zip(got, want):
+            np.testing.assert_array_equal(a, b)
+        assert c == counts, (refill, c, counts)
+    assert 0.02 < want[2].mean() < 0.98
+    e.close()
