@@ -326,9 +326,9 @@ __device__ __forceinline__ void set_ray(RayState& r, f3 org, f3 d)
 // or cells it steps into are empty, so that more lanes reach candidates by the
 // wave's test batch.
 //
-// These kernels are bound by VALU issue under divergence (81 % busy at 38 % of
-// the lanes on the 1M-triangle AO frame), so what counts is instructions per
-// iteration.  An item's owner is found without a list of items: a lane writes its number
+// These kernels are bound by VALU issue under divergence (83 % busy at 48 % of
+// the lanes on the 1M-triangle AO frame; 81 % at 38 % before the following), so
+// what counts is instructions per iteration.  An item's owner is found without a list of items: a lane writes its number
 // at its first item's place in 64 words of LDS, and a maximum scan over the
 // wave carries it to the lane's other items (the owners increase with the
 // items); the item's candidate is its place plus its owner's offset.  One LDS
@@ -337,7 +337,8 @@ __device__ __forceinline__ void set_ray(RayState& r, f3 org, f3 d)
 // multiplies) and the short reciprocals: AO kernel of that frame 2.29 -> 2.12
 // ms, heightfield 1024x768 camera rays 0.54 -> 0.42 and paths 0.85 -> 0.68 ms,
 // 250,000 paths on a uniform grid 1.45 -> 1.17 ms.  4M rays in random order on
-// 102,400 triangles stay at 1.5 ms: the L2's lines bound them, not the VALU.
+// 102,400 triangles stay at 1.5 ms: lines from beyond the L2 bound them (7.5 GB a
+// launch at 5.8 TB/s), not the VALU.
 constexpr int kBatchK = 12;   // candidates a lane hands to its wave per iteration
 
 // Rays per wave of a launch of n rays that should spread over `blocks`

@@ -430,6 +430,9 @@ void launch_path_multi(const TraceScene& S, const CameraDev& cam, const RenderAr
 {
     const uint32_t npix = (uint32_t)cam.res_x * (uint32_t)cam.res_y;
     const dim3 g(blocks_for(npix)), b(kBlock);
+    // all the waves that fit for the paths, half of them for the shadow rays:
+    // paths of 160x120 on 82,000 triangles 288 us a frame so, 298 / 316 / 344 with
+    // half, a quarter and full waves (three contexts in turn 106 / 108 / 116 / 125)
     const uint32_t pl = wave_lanes(npix, 4 * device_cus()), sl = wave_lanes(npix, 2 * device_cus());
     const dim3 gp(wave_blocks(npix, pl)), gs(wave_blocks(npix, sl));
     if (S.two_level) {

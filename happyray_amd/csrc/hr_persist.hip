@@ -206,11 +206,15 @@ struct RayFetch {
 
 // Rays per wave and workgroups of a launch of n rays, and the rays of a run: an
 // eighth of a wave's share in whole waves, at most 256.  The counter's atomics
-// serialise at the memory side (12 ns each): 8.4M AO rays fetched 56 at a time
-// made 150,000 of them in 2 ms.  AO of 1M triangles 1.953 ms fetching what is
-// idle, 1.950 in runs of 64, 1.760 in runs of 128.  Where an eighth of the share
-// is less than a wave (1M rays: 20) what is idle is fetched (chunk 0): waves that
-// keep rays to start at the end of the launch cost more (0.93 -> 1.00 ms).
+// serialise at the memory side (12 ns each), which bounds short coherent rays:
+// 8.4M AO rays fetched 56 at a time made 150,000 of them in 2 ms.  AO of 1M
+// triangles 1.953 ms fetching what is idle, 1.950 in runs of 64, 1.760 in runs of
+// 128; 7M camera rays over 64 scenes 1.82 / 1.49 / 0.95 / 0.93 ms idle / 64 / 128 /
+// 256.  Random rays pay for the waves that keep rays to start at the launch's end:
+// 4M closest 3.08 / 3.19 / 3.31 / 3.38 ms, 14M 10.36 / 10.49 / 10.58 / 10.75, 4M
+// occlusion 1.56 / 1.58 / 1.57 / 1.59.  Where an eighth of the share is less than a
+// wave (below 3.1M rays) what is idle is fetched (chunk 0): 1M closest 0.91 / 0.97 /
+// 1.11 / 1.19.
 struct RayLaunch {
     uint32_t lanes, blocks, refill, chunk;
     bool pooled;
@@ -219,8 +223,9 @@ struct RayLaunch {
 inline RayLaunch ray_launch(uint32_t n, uint32_t blocks_max, uint32_t refill)
 {
     RayLaunch l;
-    // one wave per SIMD: 4096 occlusion rays take 59 us so, 92 and 161 us with two
-    // and six waves of fewer rays; 1,000 rays of one per wave 52 us (64: 78 us)
+    // one wave per SIMD: 4096 occlusion rays take 30 us so, 38 and 50 us with two
+    // and four waves of fewer rays, 55 us with 64 a wave; 1,000 closest hits 57 us
+    // (64 a wave: 112).  Three contexts in turn 12 / 14 / 17 / 20 us, and 22 (40)
     l.lanes = wave_lanes(n, device_cus());
     const uint32_t need = wave_blocks(n, l.lanes);
     l.pooled = need > blocks_max;

@@ -355,7 +355,8 @@ typedef struct {
                                   tests its own candidates (fuse_units applies).  Same
                                   results and work statistics; with 1 an any-hit ray may
                                   test up to 11 candidates past its first hit, which the
-                                  statistics leave out                                  */
+                                  statistics leave out.  The multi-kernel path tracer
+                                  (mode 1) takes it as 1                                 */
     int advance_steps;         /* test_batch 1: grid steps a lane may take per loop
                                   iteration to reach its next candidates, 1..4 (default 2) */
     int frame_lanes;           /* captured frames: 2 (default) two lanes of per-frame
