@@ -224,7 +224,7 @@ def test_paths_of_several_contexts_share_the_gpu(mesh, kind, density):
 
     small, large = rate(80000), rate(240000)
     print(f"paths/us: {small * 1e-6:.0f} at 80,000 a launch, {large * 1e-6:.0f} at 240,000", flush=True)
-    assert small > 0.63 * large
+    assert small > 0.6 * large
 
 
 # the flat kernel has at most six workgroups per CU, so rays past 393,216 come
