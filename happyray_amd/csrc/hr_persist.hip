@@ -277,7 +277,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8))) voi
                 if (j < nrays) {
                     const bool ok = gen.start(j, r, S);
                     started += ok ? 1u : 0u;
-                    live = ok && ray_begin<kTwo, kAny>(G, S, r, wk);
+                    live = ok && ray_begin<kTwo, kAny, false, true>(G, S, r, wk);
                     if (!live) gen.finish(j, r, ok, S);
                 }
             }
@@ -290,11 +290,11 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8))) voi
             bool done = false;
             if (kFuse) {
                 if (r.it >= r.end)
-                    done = kTwo ? !advance_two_level<kAny>(G, S, r, wk) : !advance_uniform<kAny>(G, S, r, wk);
+                    done = kTwo ? !advance_two_level<kAny>(G, S, r, wk) : !advance_uniform_cells<kAny>(G, S, r, wk);
                 if (!done && r.it < r.end) done = test_one<kAny>(S, r, wk);
             } else {
                 if (r.it < r.end) done = test_one<kAny>(S, r, wk);
-                else done = kTwo ? !advance_two_level<kAny>(G, S, r, wk) : !advance_uniform<kAny>(G, S, r, wk);
+                else done = kTwo ? !advance_two_level<kAny>(G, S, r, wk) : !advance_uniform_cells<kAny>(G, S, r, wk);
             }
             if (done) {
                 live = false;
